@@ -18,7 +18,15 @@ __device__ __forceinline__ float silu_f(float v) { return v / (1.0f + expf(-v));
 
 // ---- fp32 product on bf16 MFMA: every operand as the sum of three bf16 terms ----
 // v = h + m + l with h = bf16(v), m = bf16(v - h), l = bf16(v - h - m): 3 x 8
-// significant bits hold all 24 of v, so the three terms add up to v exactly.
+// significant bits hold all 24 of v, so the three terms add up to v exactly,
+// unless they leave bf16's range.  The last bit of v = 2^e (1 + ...) has weight
+// 2^(e - 23), and bf16 holds multiples of 2^-133, so below 2^-110 the low terms
+// would lose bits; every operand is therefore multiplied by SPLIT_SCALE first
+// (exact), which lifts the last bit of the smallest fp32 number, 2^-149, to
+// 2^-133, and the sums are divided by SPLIT_SCALE^2 at the end (one rounding,
+// where the result is subnormal).  What that costs at the other end: a value
+// of 2^112 or a sum of 2^96 and more overflows, and is computed otherwise (see
+// split_tile).
 // A product a b is then the six term products of order 2^0 (ah bh), 2^-9 (ah
 // bm, am bh) and 2^-18 (am bm, ah bl, al bh) relative to it; the three left
 // out (am bl, al bm, al bl) are below 2^-26, under the rounding of an fp32
@@ -26,6 +34,7 @@ __device__ __forceinline__ float silu_f(float v) { return v / (1.0f + expf(-v));
 // the bfloat16 artificial intelligence datatype for higher-precision
 // computations", 2019.)  Six v_mfma_f32_32x32x16_bf16 take 192 cycles where
 // eight v_mfma_f32_32x32x2f32 take 512.
+constexpr float SPLIT_SCALE = 0x1p16f;
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
@@ -38,6 +47,8 @@ __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
 }
 __device__ __forceinline__ void split2(float a, float b, Split8& o, int p) {   // values 2 p, 2 p + 1
+    a *= SPLIT_SCALE;
+    b *= SPLIT_SCALE;
     const uint32_t h = pack_bf16(a, b);
     const float ra = a - __uint_as_float(h << 16), rb = b - __uint_as_float(h & 0xffff0000u);
     const uint32_t m = pack_bf16(ra, rb);
@@ -59,15 +70,18 @@ __device__ __forceinline__ f32x16 mfma_bf16(u32x4 a, u32x4 b, f32x16 c) {
 //    quad of lanes touches four rows of A: 20.7 us at 1024^3 on 17.7.)
 //    16-byte chunk c of A row r sits in slot c ^ ((r / 4) % 4), so that 16
 //    lanes reading 16 rows touch 16 distinct bank groups;
-//  * reads unit t+2 into registers, splits unit t+1 (176 vector instructions)
+//  * reads unit t+2 into registers, splits unit t+1 (208 vector instructions)
 //    and runs the 24 MFMAs of unit t in one straight-line block; a
 //    v_mfma_f32_32x32x16_bf16 hides six of the split's instructions (a
-//    16x16x32 two, and each one more costs four cycles).
+//    16x16x32 two, and each one more costs four cycles).  32 of the 208 are
+//    the scaling: 1024^3 14.4 -> 14.6 us, 2048^3 97.4 -> 99.2, 512 x 512 x 2048
+//    20.8 -> 22.0, 32x56x56x64 3x3 convolution 55.8 -> 56.4 (a check of the
+//    operands for small values would have to look at every element as well).
 // 229 registers and 64 KB of LDS: two workgroups per CU, whose instructions
 // interleave (one wave alone issues one per four to five cycles: 17.7 us at
 // 1024^3) and whose first fetches and last sums overlap.  With eight waves per
 // workgroup and one workgroup per CU: 15.4 us at 1024^3 and 27.0 at 2048 x
-// 2048 x 256; as here 14.5 and 19.3 (18.2 and 24.8 on fp32 MFMA).  What
+// 2048 x 256; as here 14.4 and 19.6 (17.8 and 24.5 on fp32 MFMA).  What
 // bounds a long K is power: at 1024 x 1024 x 4096 zeros run in 35 us and
 // uniform operands in 51 (without the split's instructions 40, without DMA 44).
 // The operand layout in k is lane half h = k 4 h .. 4 h + 3 and 8 + 4 h ..
@@ -76,16 +90,15 @@ __device__ __forceinline__ f32x16 mfma_bf16(u32x4 a, u32x4 b, f32x16 c) {
 // Any shape and alignment: rows past M read row M - 1, and what lies past the
 // end of an operand reads as zero (a raw buffer checks every dword); results
 // past the output are not stored.  k past K is zero in B, and masked in A.
-// The split cannot hold an infinity (inf - inf), nor the low terms of values
-// near the smallest bf16 (2^-126).  A tile with a sum that is not finite, or
-// with an A row or B column whose values are all under 2^-95 and not all zero,
-// is computed again by v_mfma_f32_32x32x2f32 from the unsplit operands.  (A
-// row's exponents are gathered by OR over its h terms: a field of 32 or more in
-// the OR means a value of 2^-95 or more.  Nearly always a wave's first unit
-// shows that for every row and column; gathered over all units it took 1.5 us
-// of 16 at 1024^3.)
-// 1021 x 1531 x 2043: 44 us (138 with element-wise loads on fp32 MFMA); 2048^3
-// 94 us (125); 1024 x 2048 x 4096 97 us (120).
+// The split cannot hold an infinity (inf - inf) nor what SPLIT_SCALE lifts past
+// the largest number: a tile with a sum that is not finite is computed again by
+// v_mfma_f32_32x32x2f32 from the unsplit, unscaled operands.  That second pass
+// takes as long as a product on fp32 MFMA: 1024^3 with an infinity in one row of
+// A 32.7 us (its row of tiles twice, the others waiting for it), 2048^3 with
+// all sums past 2^96 222 us (99; 133 on fp32 MFMA alone).
+// 1021 x 1531 x 2043: 47 us (138 with element-wise loads on fp32 MFMA); 2048^3
+// 99 us (133); 1024 x 2048 x 4096 97 us (127); all launches back to back on one
+// set of operands.
 constexpr uint32_t SP_BAND = 4;          // tile-rows per XCD band (xcd_band_tile)
 constexpr int SP_W = 4;                 // waves per workgroup
 constexpr uint32_t SP_SLOT = 8192;       // one unit of A and B
@@ -106,8 +119,6 @@ __device__ __forceinline__ void split_tile(const SplitTile& g, DmaA dma_a) {
     constexpr bool DUAL = EPI == EPI_SWIGLU;
     __shared__ __attribute__((aligned(1024))) uint8_t L[SP_W * SP_WAVE];
     __shared__ float rss[SP_W][64];      // RMS: wave, row
-    __shared__ uint32_t ors[SP_W][4][64];   // wave, A rows li and 32 + li, B columns of block 0 and 1
-    __shared__ uint32_t sure[SP_W];
     __shared__ uint32_t flag[SP_W];
 
     const uint32_t tid = threadIdx.x, lane = tid & 63;
@@ -230,21 +241,6 @@ __device__ __forceinline__ void split_tile(const SplitTile& g, DmaA dma_a) {
                                       t == 1 ? y.l : t == 2 || t == 4 ? y.m : y.h, acc[i][j]);
             }
     };
-    // OR of the h terms multiplied so far: A blocks 0, 1, B blocks 0, 1.  When
-    // the wave's first unit shows that no row or column of the tile is tiny
-    // (`unsure` false), the other units are not looked at.
-    constexpr uint32_t TINY = 32 << 7;   // bf16 bits of 2^-95
-    uint32_t bits[4] = {};
-    bool unsure = true;
-    auto top = [](uint32_t v) { return (v | v >> 16) & 0x7fffu; };
-    auto gather = [&](const Ops& o) {
-#pragma unroll
-        for (int x = 0; x < 4; ++x) {
-            const u32x4 h = x < 2 ? o.a[x].h : o.b[x - 2].h;
-            bits[x] |= h[0] | h[1];
-            bits[x] |= h[2] | h[3];
-        }
-    };
     auto clear = [&] {
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
@@ -254,9 +250,10 @@ __device__ __forceinline__ void split_tile(const SplitTile& g, DmaA dma_a) {
         }
     };
     // The four waves' partials meet in LDS, each in its wave's own ring.
-    // Wave w finishes 64 / SP_W rows of both column blocks. `check`: true in every thread, with nothing stored, if a sum of
-    // the tile is not finite or an operand row is tiny.
-    auto finish = [&](bool check) -> bool {
+    // Wave w finishes 64 / SP_W rows of both column blocks.  `scaled`: the sums are
+    // those of split operands; true in every thread, with nothing stored, if one of
+    // the tile's is not finite.
+    auto finish = [&](bool scaled) -> bool {
         auto part = [&](uint32_t w) { return reinterpret_cast<float*>(L + w * SP_WAVE); };
 #pragma unroll
         for (int ij = 0; ij < 4; ++ij)
@@ -268,12 +265,6 @@ __device__ __forceinline__ void split_tile(const SplitTile& g, DmaA dma_a) {
                 const float t = ss[i] + __shfl_xor(ss[i], 32);
                 if (lh == 0) rss[wave][32 * i + li] = t;
             }
-        }
-        if (check) {
-            if (unsure)
-#pragma unroll
-                for (int x = 0; x < 4; ++x) ors[wave][x][lane] = bits[x];
-            if (lane == 0) sure[wave] = !unsure;
         }
         __syncthreads();
         constexpr int QN = 32 / SP_W;   // accumulator registers finished per wave and block
@@ -294,16 +285,7 @@ __device__ __forceinline__ void split_tile(const SplitTile& g, DmaA dma_a) {
                 odd |= (gr < M) & (gc < N) & !(fabsf(t) <= 3.402823466e38f);
             }
         }
-        if (check) {
-            uint32_t any_sure = 0;
-#pragma unroll
-            for (int w = 0; w < SP_W; ++w) any_sure |= sure[w];
-            if (!any_sure && tid < 128) {
-                uint32_t t = 0;
-#pragma unroll
-                for (int w = 0; w < SP_W; ++w) t |= ors[w][tid >> 5][li] | ors[w][tid >> 5][32 + li];
-                odd |= top(t) - 1 < TINY - 1;   // tiny and not all zero
-            }
+        if (scaled) {
             const bool any = __builtin_amdgcn_ballot_w64(odd) != 0;
             if (lane == 0) flag[wave] = any;
             __syncthreads();
@@ -322,12 +304,12 @@ __device__ __forceinline__ void split_tile(const SplitTile& g, DmaA dma_a) {
 #pragma unroll
         for (int q = 0; q < QN; ++q) {
             const uint32_t lr = 32 * i + 8 * ((q0 + q) >> 2) + 4 * lh + (q & 3), gr = m0 + lr;
-            float sc = 1.0f;
+            float sc = scaled ? 1.0f / (SPLIT_SCALE * SPLIT_SCALE) : 1.0f;
             if (RMS) {
                 float t = 0.f;
 #pragma unroll
                 for (int w = 0; w < SP_W; ++w) t += rss[w][lr];
-                sc = rsqrtf(t / (float)K + g.eps);
+                sc *= rsqrtf(t / (float)K + g.eps);
             }
 #pragma unroll
             for (int j = 0; j < (DUAL ? 1 : 2); ++j) {
@@ -358,9 +340,6 @@ __device__ __forceinline__ void split_tile(const SplitTile& g, DmaA dma_a) {
         mask_top(r[0]);
         split(r[0], o[0]);
         pin(o[0]);
-        gather(o[0]);
-        unsure = __builtin_amdgcn_ballot_w64(min(min(top(bits[0]), top(bits[1])),
-                                                 min(top(bits[2]), top(bits[3]))) < TINY) != 0;
         if (n > 2) {
             dma(0, 2);
             asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NA + 4) : "memory");
@@ -372,7 +351,6 @@ __device__ __forceinline__ void split_tile(const SplitTile& g, DmaA dma_a) {
             constexpr int c = decltype(c_)::value;
             asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
             if (t + 3 < n) dma((c ^ 1) * SP_SLOT, t + 3);
-            if (unsure && t > 0) gather(o[c]);
             __builtin_amdgcn_sched_barrier(0);
             read(r[c], c * SP_SLOT);
             if (RMS) { ss[0] += ss_next[0]; ss[1] += ss_next[1]; }
@@ -383,7 +361,7 @@ __device__ __forceinline__ void split_tile(const SplitTile& g, DmaA dma_a) {
             for (int x = 0; x < 24; ++x) {
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
                 __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, 9, 0);
             }
             __builtin_amdgcn_sched_barrier(0);
         };

@@ -120,3 +120,21 @@ def test_conv2d_values_the_split_cannot_hold(mb, dev, n, c):
     assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
     fin = np.isfinite(want)
     assert np.all(np.abs(got[fin] - want[fin]) <= (2.0 ** -20 * size)[fin])
+
+
+@pytest.mark.parametrize("c", [4, 3, 64])
+def test_conv2d_small_weights_keep_their_bits(mb, dev, c):
+    """A patch that a ReLU left at zero except under one tiny weight: the outputs are
+    that product alone, exact up to one rounding (the bound leaves room for one more)."""
+    n, h, w, o = 32, 56, 56, 64
+    x = torch.zeros((n, h, w, c))
+    x[..., 1] = seeded(1, (n, h, w)).clamp_min(0) * 1e30
+    wt = seeded(2, (o, 3, 3, c))
+    wt[..., 1] = 0.0
+    wt[:, 1, 1, 1] = 1.37 * 2.0 ** -torch.arange(100, 100 + o).clamp_max(126).float()
+    d_x, d_w = x.to(dev), wt.to(dev)
+    d_y = torch.zeros((n, h, w, o), device=dev)
+    launch("mb_launch_conv2d_nhwc_f32", ptr(d_x), ptr(d_w), ptr(d_y), n, h, w, c, o, 3, 3, 1, 1, None)
+    want = x[..., 1].numpy().astype(np.float64)[..., None] * wt[:, 1, 1, 1].numpy().astype(np.float64)
+    # (a product below the smallest normal number is rounded to a multiple of 2^-149)
+    assert np.all(np.abs(d_y.cpu().numpy() - want) <= 2.0 ** -22 * want + 2.0 ** -149)

@@ -141,3 +141,40 @@ def test_matmul_f32_operand_past_2gb(mb, dev):
     want = oracle.matmul(a[rows].cpu().numpy(), b.cpu().numpy())
     assert_close(c[rows].cpu().numpy(), want, 1e-4, 1e-4, "past 2 GB")
     assert torch.isfinite(c).all()
+
+
+# Elements far below the rest of their row or column, and alone in a product: every
+# term of the split has to survive, whatever stands beside it.
+@pytest.mark.parametrize("e", [-100, -110, -115, -120, -126, -130, -140, -149])
+def test_matmul_f32_small_elements_keep_their_bits(mb, dev, e):
+    """A = [1, v], B = [0; w]: the product v w alone, v from 2^e on and w = 2^100 (or the
+    other way round).  Both are powers of two or 24-bit numbers, so fp32 products would
+    be exact up to one rounding; a subnormal v has the bits fp32 holds."""
+    v = np.float32(1.37 * 2.0 ** e)
+    for n in (1, 2, 65):
+        a = torch.tensor([[1.0, float(v)]])
+        b = torch.zeros((2, n))
+        b[1] = 2.0 ** 100
+        want = float(v) * 2.0 ** 100
+        for x, y in ((a, b), (b.T.contiguous(), a.T.contiguous())):
+            d_x, d_y = x.to(dev), y.to(dev)
+            m, nn = x.shape[0], y.shape[1]
+            d_c = torch.zeros((m, nn), device=dev)
+            launch("mb_launch_matmul_f32", ptr(d_x), ptr(d_y), ptr(d_c), m, nn, 2, None)
+            got = d_c.cpu().numpy().astype(np.float64)
+            assert np.all(np.abs(got - want) <= 2.0 ** -23 * want), (n, got.ravel()[0] / want - 1)
+
+
+@pytest.mark.parametrize("m,n,k", [(70, 67, 129), (128, 192, 640)])
+@pytest.mark.parametrize("scale", [1e-30, 1e-35, 1e-37])
+def test_matmul_f32_mixed_magnitudes(mb, dev, m, n, k, scale):
+    """One ordinary value in every row, met by a zero; the others carry the sum."""
+    a, b = seeded(7, (m, k)) * scale, seeded(8, (k, n)) * 1e30
+    a[:, 0], b[0] = 1.0, 0.0
+    for x, y in ((a, b), (b.T.contiguous(), a.T.contiguous())):
+        mm, nn = x.shape[0], y.shape[1]
+        d_x, d_y = x.to(dev), y.to(dev)
+        d_c = torch.zeros((mm, nn), device=dev)
+        launch("mb_launch_matmul_f32", ptr(d_x), ptr(d_y), ptr(d_c), mm, nn, k, None)
+        X, Y = x.numpy().astype(np.float64), y.numpy().astype(np.float64)
+        assert np.all(np.abs(d_c.cpu().numpy() - X @ Y) <= 2.0 ** -22 * (np.abs(X) @ np.abs(Y)))

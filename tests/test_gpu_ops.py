@@ -238,3 +238,73 @@ def test_rejects_bad_shapes(mb):
     with pytest.raises(native.NativeError):   # odd D
         run_bound("rope_embedding_f32", [(0, seeded(43, (3, 5)))], [(1, (3, 5))],
                   [(2, "u32", 3), (3, "u32", 5), (4, "f32", 10000.0)])
+
+
+def _silu(v):
+    return v / (1 + np.exp(-v))
+
+
+@pytest.mark.parametrize("scale", [1.0, 1e-36])
+@pytest.mark.parametrize("m,n,k", [(70, 67, 129), (130, 64, 640)])
+def test_fused_products_of_values_the_split_cannot_hold(mb, m, n, k, scale):
+    """The row scale, residual and SwiGLU epilogues over bf16 term products: rows of
+    elements of size `scale` and one ordinary value that meets zeros, and (scale 1)
+    an infinite weight, whose tile is multiplied a second time.  Sums are within
+    2^-21 of the products' magnitudes (2^-22 and the row scale's rounding)."""
+    x = seeded(60, (m, k)) * scale
+    x[:, 0] = 1.0
+    wg, wu = seeded(61, (k, n)) / scale, seeded(62, (k, n)) / scale
+    wg[0], wu[0] = 0.0, 0.0
+    if scale == 1.0:
+        wu[5, 3] = float("inf")
+    X, G, U = f64(x), f64(wg), f64(wu)
+    inf = np.isinf(U).any(0)
+    Uf = np.where(np.isinf(U), 0, U)
+    xn = oracle.rms_norm(X, 1e-5)
+
+    def near(got, want, bound):
+        assert np.array_equal(got[:, inf], want[:, inf])
+        assert np.all((np.abs(got - want) <= bound)[:, ~inf])
+
+    (y,) = run_bound("rms_norm_linear_f32", [(0, x), (1, wu.T.contiguous())], [(2, (m, n))],
+                     [(3, "u32", m), (4, "u32", n), (5, "u32", k), (6, "f32", 1e-5)])
+    with np.errstate(all="ignore"):
+        near(f64(y), xn @ U, 2.0 ** -21 * (np.abs(xn) @ np.abs(Uf)))
+
+    # SwiGLU: silu's slope is at most 1.1; its exponential and division round a few times
+    (y,) = run_bound("swiglu_f32", [(0, x), (1, wg), (2, wu)], [(3, (m, n))],
+                     [(4, "u32", m), (5, "u32", n), (6, "u32", k)])
+    g, u = X @ G, X @ Uf
+    size = 1.1 * (np.abs(X) @ np.abs(G)) * np.abs(u) + np.abs(_silu(g)) * (np.abs(X) @ np.abs(Uf))
+    with np.errstate(all="ignore"):
+        near(f64(y), _silu(g) * (X @ U), 2.0 ** -21 * size + 2.0 ** -20 * np.abs(_silu(g) * u))
+
+
+@pytest.mark.parametrize("scale", [1.0, 1e-36])
+def test_layer_products_of_values_the_split_cannot_hold(mb, scale):
+    """The prefill layer with W_o = 0: x + act W_down, where W_down's elements are of
+    size `scale` but for one row of ones that meets zero activations, and (scale 1)
+    hold an infinity.  70 x 576 x 576, 70 x 644 x 576 and 70 x 576 x 644 products."""
+    s, d, h, hkv, ff = 70, 576, 9, 3, 644
+    x, wq, _ = _attn_inputs(s, d, h, hkv, 70)
+    wgu, wd = seeded(73, (d, 2 * ff)) * d ** -0.5, seeded(74, (ff, d)) * scale
+    wgu[:, ff:] /= scale
+    wgu[:, ff], wd[0] = 0.0, 1.0
+    if scale == 1.0:
+        wd[5, 9] = float("inf")
+    (y,) = run_bound("llama_decoder_layer_f32",
+                     [(0, x), (1, wq), (2, torch.zeros(d, d)), (3, wgu), (4, wd)], [(5, (s, d))],
+                     [(6, "u32", s), (7, "u32", d), (8, "u32", h), (9, "u32", hkv),
+                      (10, "u32", ff), (11, "f32", 10000.0), (12, "f32", 1e-5)])
+    X, G, D = f64(x), f64(wgu), f64(wd)
+    inf = np.isinf(D).any(0)
+    Df = np.where(np.isinf(D), 0, D)
+    xn = oracle.rms_norm(X, 1e-5)
+    g, u = xn @ G[:, :ff], xn @ G[:, ff:]
+    act = _silu(g) * u
+    size = np.abs(xn) @ np.abs(G)
+    d_act = 2.0 ** -21 * (1.1 * size[:, :ff] * np.abs(u) + np.abs(_silu(g)) * size[:, ff:]) + 2.0 ** -20 * np.abs(act)
+    want, got = X + act @ Df, f64(y)
+    bound = d_act @ np.abs(Df) + 2.0 ** -22 * (np.abs(act) @ np.abs(Df)) + 2.0 ** -23 * np.abs(want)
+    assert np.all((np.abs(got - want) <= bound)[:, ~inf])
+    assert np.array_equal(got[:, inf], np.sign(act[:, 5:6]) * np.inf * np.ones((1, inf.sum())))
