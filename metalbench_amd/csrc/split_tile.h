@@ -137,6 +137,10 @@ __device__ __forceinline__ void split_tile(const SplitTile& g, DmaA dma_a) {
     // DMA instruction i of a unit: B^T rows 16 i + lane / 4, slot lane % 4; B k-rows 4 i + lane / 16 (DUAL: LDS row 8 (i % 2) + lane / 8 of
     // gate, then up; k-row r sits in row r ^ ((r / 4) % 2), so that the k-rows
     // of the two half-waves, r and r + 4, lie in opposite halves of the banks).
+    // k-rows past K lie past the end of B, and are at most 15: under 2^32 bytes
+    // together with K < 2^31 / (4 ldb) of them when K is 16 or more.  With K
+    // below 16 a row of very many columns would wrap around, and takes an
+    // out-of-range offset.
     uint32_t b_vo[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -144,8 +148,12 @@ __device__ __forceinline__ void split_tile(const SplitTile& g, DmaA dma_a) {
         if (BL == BL_NK) b_vo[i] = (min(n0 + r, N - 1) * ldb + 4 * ch) * 4;
         else if (DUAL) {
             const uint32_t p = 8 * (i & 1) + (lane >> 3);
-            b_vo[i] = ((p ^ ((p >> 2) & 1)) * ldb + n0 + 4 * (lane & 7)) * 4;
-        } else b_vo[i] = ((4 * i + (lane >> 4)) * ldb + n0 + 4 * (lane & 15)) * 4;
+            const uint32_t k = p ^ ((p >> 2) & 1);
+            b_vo[i] = k < K ? (k * ldb + n0 + 4 * (lane & 7)) * 4 : 0x80000000u;
+        } else {
+            const uint32_t k = 4 * i + (lane >> 4);
+            b_vo[i] = k < K ? (k * ldb + n0 + 4 * (lane & 15)) * 4 : 0x80000000u;
+        }
     }
     // the wave takes units u = wave (mod SP_W), last first
     const uint32_t units = (K + 15) / 16;

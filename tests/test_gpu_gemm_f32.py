@@ -178,3 +178,26 @@ def test_matmul_f32_mixed_magnitudes(mb, dev, m, n, k, scale):
         launch("mb_launch_matmul_f32", ptr(d_x), ptr(d_y), ptr(d_c), mm, nn, k, None)
         X, Y = x.numpy().astype(np.float64), y.numpy().astype(np.float64)
         assert np.all(np.abs(d_c.cpu().numpy() - X @ Y) <= 2.0 ** -22 * (np.abs(X) @ np.abs(Y)))
+
+
+@pytest.mark.parametrize("dual", [False, True])
+def test_matmul_f32_very_wide_rows(mb, dev, dual):
+    """15 rows of this B are just over 2^32 bytes: k-rows past K must read as zero, not
+    wrap around to B's start, where an infinity stands that column 100 does not have."""
+    n = 71_600_000
+    at = (15 * n) % 2 ** 30 + 100       # what column 100 of row 15 would wrap to
+    a = torch.full((1, 1), 2.0, device=dev)
+    b = torch.ones((1, n), device=dev)
+    b[0, at] = float("inf")
+    c = torch.zeros((1, n), device=dev)
+    if dual:                            # SwiGLU: silu(a b) (a b)
+        binds = [mb.make_binding(i, mb.ROLE_INPUT if i < 3 else mb.ROLE_OUTPUT, "f32", t.data_ptr(), t.numel() * 4)
+                 for i, t in enumerate((a, b, b, c))]
+        binds += [mb.make_binding(4 + i, mb.ROLE_SCALAR, "u32", value=v) for i, v in enumerate((1, n, 1))]
+        mb.run(mb.kernel_find("swiglu_f32"), binds, 0, 1)
+    else:
+        launch("mb_launch_matmul_f32", ptr(a), ptr(b), ptr(c), 1, n, 1, None)
+    want = 4.0 / (1.0 + float(np.exp(-2.0))) if dual else 2.0
+    assert torch.isinf(c[0, at])
+    c[0, at] = want
+    assert (c - want).abs().max().item() <= 1e-6 * want
