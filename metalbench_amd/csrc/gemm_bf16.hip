@@ -22,7 +22,8 @@
 //    tile leaves CUs idle below 256 tiles, and unaligned rows were loaded element
 //    by element: 1000 x 3000 x 4096 159 -> 36 us, 1001 x 3001 x 4095 457 -> 71,
 //    128 x 4096 x 4096 148 -> 15, 64 x 512 x 4096 142 -> 7.4;
-//  * operands or results past 2 GB that are not full tiles, and K = 0, take
+//  * operands or results past 2 GB that are not full tiles, more than 16 million
+//    columns with K < 128, and K = 0 take
 //    gemm_bf16_kernel (4 x 4 v_mfma_f32_32x32x16_bf16 per wave), BK = 64 with an LDS
 //    double buffer:
 //    both operands stored K-contiguous, row pitch 72 bf16 (144 B), 2 x 2 x
@@ -1226,9 +1227,11 @@ int launch_gemm_bf16(const uint16_t* a, const uint16_t* b, uint16_t* c, uint32_t
     if (nblocks > 0x7fffffffull) return fail(MB_E_ARG, "matmul_bf16: shape too large");
     const bool aligned = (k % 8 == 0) && (n % 8 == 0) &&
                          ((((uintptr_t)a) | ((uintptr_t)b)) & 15) == 0;
-    // 32-bit buffer offsets reach every operand
+    // 32-bit buffer offsets reach every operand, and B's k-rows up to the next multiple
+    // of 128 (the deepest stage) without wrapping around to its start
     const bool near = k > 0 && (uint64_t)m * k * 2 < (1ull << 31) && (uint64_t)k * n * 2 < (1ull << 31) &&
-                      (uint64_t)m * n * 2 < (1ull << 31);
+                      (uint64_t)m * n * 2 < (1ull << 31) &&
+                      (((uint64_t)k + 127) & ~127ull) * n * 2 < (1ull << 32);
     // Full 256 x 256 tiles, more than 64 of them (or a C past 2 GB).  Up to 64, one
     // round of tiles a quarter as large or smaller is faster (512 x 6144 x 4096: 66
     // us on 48 tiles, 36 on 256; 2048^3: 37 and 22); from 65 it takes two rounds (2048 x

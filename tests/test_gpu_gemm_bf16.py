@@ -154,3 +154,18 @@ def test_matmul_bf16_operand_past_2gb(mb, dev):
         want = oracle.matmul(oracle.as_f64(a[rows]), oracle.as_f64(b))
         assert_close(oracle.as_f64(c[rows]), want, 1e-2, 1e-3, f"past 2 GB, k {k}")
         assert torch.isfinite(c).all()
+
+
+def test_matmul_bf16_very_wide_rows(mb, dev):
+    """24 rows of this B are just over 2^32 bytes: k-rows past K must read as zero, not
+    wrap around to B's start, where an infinity stands that column 100 does not have."""
+    n, k = 89_500_000, 2
+    at = (24 * n) % 2 ** 31 + 100       # what column 100 of row 24 would wrap to
+    a = torch.ones((1, k), device=dev, dtype=torch.bfloat16)
+    b = torch.ones((k, n), device=dev, dtype=torch.bfloat16)
+    b[0, at] = float("inf")
+    c = torch.zeros((1, n), device=dev, dtype=torch.bfloat16)
+    launch("mb_launch_matmul_bf16", ptr(a), ptr(b), ptr(c), 1, n, k, None)
+    assert torch.isinf(c[0, at])
+    c[0, at] = 2.0
+    assert (c == 2.0).all()
