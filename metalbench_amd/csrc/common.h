@@ -120,6 +120,7 @@ static inline uint32_t cdiv(uint32_t a, uint32_t b) { return (a + b - 1) / b; }
 // C[b] = A[b] @ B[b] (row-major, leading dimensions lda/ldb/ldc), batch b at
 // blockIdx.y with element strides batch_*.  Kinds:
 //   PLAIN       C = A B
+//   PLAIN_MFMA  C = A B, full tiles on fp32 MFMA
 //   RMS         C = rmsnorm(A) B            (row scale rsqrt(mean(A_row^2) + eps), K = row length)
 //   RMS_BT      C = rmsnorm(A) B^T, B [N][K]
 //   RESID       C = A B + R                 (R [M][N], leading dimension ldr)
@@ -136,8 +137,8 @@ struct GemmF32Args {
     float eps;
 };
 enum GemmF32Kind {
-    GEMM_F32_PLAIN, GEMM_F32_RMS, GEMM_F32_RMS_BT, GEMM_F32_RESID, GEMM_F32_SWIGLU,
-    GEMM_F32_RMS_SWIGLU
+    GEMM_F32_PLAIN, GEMM_F32_PLAIN_MFMA, GEMM_F32_RMS, GEMM_F32_RMS_BT, GEMM_F32_RESID,
+    GEMM_F32_SWIGLU, GEMM_F32_RMS_SWIGLU
 };
 // ---- global -> LDS DMA ------------------------------------------------------
 typedef int32_t i32x4 __attribute__((ext_vector_type(4)));

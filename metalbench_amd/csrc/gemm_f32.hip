@@ -1,9 +1,10 @@
 // fp32 GEMM family on the matrix cores: C[M][N] = A[M][K] @ B (row-major), with
 // optional batching, a transposed B, an RMSNorm row scale and fused
-// epilogues.  Three kernels (64 x 64 tiles on bf16 MFMA with every operand
+// epilogues.  Four kernels (64 x 64 tiles on bf16 MFMA with every operand
 // split into three bf16 terms, for nearly all shapes; 32 x 32 tiles on fp32
-// MFMA with K spread over waves for small problems; register-staged 64 x 64
-// tiles on fp32 MFMA for operands past 2 GB) serve these registry entries:
+// MFMA with K spread over waves for small problems; 64 x 64 tiles on fp32 MFMA
+// fed by DMA for sqr_mm; register-staged ones for operands past 2 GB) serve
+// these registry entries:
 //   sqr_mm, rect_mm, fused_qkv_projection   plain C = A B
 //     (reference mlx/kernels/common/sqr_mm.py:10-11, rect_mm.py:10-11,
 //      standard/fused_qkv_projection.py:12-13; registry common/registry.py:
@@ -244,6 +245,180 @@ void gemm_f32_kernel(GemmF32Args g) {
     }
 }
 
+// C = A B on fp32 MFMA, one multiply-add per product (sqr_mm): M, N multiples of 64,
+// K a multiple of 256 and at least 512, 16-byte aligned rows, operands under 2 GB.
+// Same tile, waves and MFMA as gemm_f32_kernel<2>, but the operands go
+// global -> LDS by DMA (buffer_load ... lds) into a ring of four 64-deep k
+// stages (A 16 KB + B 16 KB each): no staging registers and no LDS store
+// instructions, whose VGPR reads held the MFMA pipe to ~72 % busy (~91 %
+// with them removed).  1024^3: 17.8 us (14.6 in bf16 terms).
+//  * A slot: [64 rows][64 k], 256-byte rows; 16-byte chunk c of row r sits in
+//    slot c ^ (r % 16), so a ds_read_b128 of 16 consecutive rows touches 16
+//    distinct bank groups;
+//  * B slot: [64 k][64 n], 256-byte k-rows; chunk c of k-row r sits in slot
+//    c ^ (8 ((r / 4) % 2)), so the two half-waves' ds_read_b32 (k-rows r and
+//    r + 4, the same 32 columns) fall in opposite halves of the bank window;
+//  * a DMA instruction writes a wave's 64 x 16 B = four rows contiguously, so
+//    lane l fetches the global chunk that its slot holds; each of the 8 waves
+//    issues 2 A and 2 B instructions per stage;
+//  * stage s (slot s % 4): groups 0-2 read the next group's operands under
+//    the current group's 4 MFMAs; before group 3 the wave waits for its DMAs
+//    of stage s+1 (vmcnt(8): stages s+2 and s+3 stay in flight), passes a
+//    barrier (every wave has read all of stage s; every wave's stage s+1 DMAs
+//    have landed), refills slot s % 4 with stage s+4 and reads stage s+1's
+//    first operands under group 3's MFMAs.
+//  * XCD-aware tile order (xcd_band_tile): at 1024^3 each XCD's 32 tiles are
+//    a band of DMA_BAND = 4 tile-rows by 8 tile-columns, which share 4 A and
+//    8 B panels in that XCD's L2 (in row-major order they shared 16 A and 2 B
+//    panels).
+constexpr int F_SLOT = BM * BK;              // floats per operand per stage slot (16 KB)
+constexpr uint32_t DMA_BAND = 4;
+
+__global__ __launch_bounds__(512)
+void gemm_f32_dma_kernel(GemmF32Args g) {
+    __shared__ __attribute__((aligned(1024))) float L[4][2 * F_SLOT];
+
+    const uint32_t tid = threadIdx.x;
+    const uint32_t lane = tid & 63;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t wk = wave >> 2, wm = (wave >> 1) & 1, wn = wave & 1;
+    uint32_t tm, tn;
+    xcd_band_tile(blockIdx.x, gridDim.x, gridDim.x / g.tiles_n, g.tiles_n, DMA_BAND, &tm, &tn);
+    const uint32_t m0 = __builtin_amdgcn_readfirstlane(tm * BM);
+    const uint32_t n0 = __builtin_amdgcn_readfirstlane(tn * BN);
+    const uint32_t K = g.k, lda = g.lda, ldb = g.ldb;
+    const uint32_t nstages = K / BK;   // a multiple of 4
+    const float* A = g.a + (size_t)blockIdx.y * g.batch_a;
+    const float* B = g.b + (size_t)blockIdx.y * g.batch_b;
+    float* C = g.c + (size_t)blockIdx.y * g.batch_c;
+
+    const i32x4 ars = dma_rsrc(A, g.m * lda * 4), brs = dma_rsrc(B, K * ldb * 4);
+    // DMA instruction i (0, 1) of wave w: rows (A) / k-rows (B) 8 w + 4 i + l/16, slot l%16.
+    const uint32_t r4 = lane >> 4, sl = lane & 15;
+    uint32_t a_voff[2], b_voff[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        a_voff[i] = (r4 * lda + 4 * (sl ^ ((8 * (wave & 1) + 4 * i + r4) & 15))) * 4;
+        b_voff[i] = (r4 * ldb + 4 * (sl ^ (8 * i))) * 4;
+    }
+    const uint32_t l0 = lds_addr(&L[0][0]);
+    auto dma = [&](int slot, uint32_t k0) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const uint32_t r = 8 * wave + 4 * i;
+            dma16(ars, l0 + slot * (8 * F_SLOT) + r * 256, a_voff[i], ((m0 + r) * lda + k0) * 4);
+            dma16(brs, l0 + slot * (8 * F_SLOT) + 4 * F_SLOT + r * 256, b_voff[i],
+                  ((k0 + r) * ldb + n0) * 4);
+        }
+    };
+
+    const uint32_t li = lane & 31, lh = lane >> 5;
+    // A operand of group gi (8 k): row wm*32 + li, chunk 2 gi + lh, swizzled.
+    const uint32_t a_row = (wm * 32 + li) * 256, a_sw = li & 15;
+    // B operand of group gi, t = 0..3: k-row 8 gi + 4 lh + t, column wn*32 + li
+    // (chunk wn*8 + li/4 ^ 8 lh, float li % 4).
+    const uint32_t b_col = 16 * ((wn * 8 + (li >> 2)) ^ (8 * lh)) + 4 * (li & 3) + 4 * lh * 256;
+    const uint8_t* l8 = reinterpret_cast<const uint8_t*>(&L[0][0]);
+    float4 a4[2], b4[2];
+    auto read_ops = [&](int slot, int gg, int c) {
+        const int gi = (int)wk * 4 + gg;
+        const uint8_t* base = l8 + slot * (8 * F_SLOT);
+        a4[c] = *reinterpret_cast<const float4*>(base + a_row + 16 * ((2 * gi + lh) ^ a_sw));
+        const float* bp = reinterpret_cast<const float*>(base + 4 * F_SLOT + 8 * gi * 256 + b_col);
+        b4[c] = make_float4(bp[0], bp[64], bp[128], bp[192]);
+    };
+    f32x16 acc = f32x16{};
+    auto mfma4 = [&](int c) {
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a4[c].x, b4[c].x, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a4[c].y, b4[c].y, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a4[c].z, b4[c].z, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a4[c].w, b4[c].w, acc, 0, 0, 0);
+    };
+    // TAIL 0: a loop stage.  TAIL 1-3: the last four stages but one, which
+    // issue no DMA (every stage they need is requested) and so wait for
+    // 8, 4 and 0 DMA instructions.  TAIL 4: the last stage (no next stage).
+    auto stage = [&](auto slot_c, auto tail_c, uint32_t s) {
+        constexpr int S = decltype(slot_c)::value;
+        constexpr int TAIL = decltype(tail_c)::value;
+#pragma unroll
+        for (int gg = 0; gg < 3; ++gg) {
+            __builtin_amdgcn_sched_barrier(0);
+            read_ops(S, gg + 1, (gg + 1) & 1);
+            mfma4(gg & 1);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (TAIL < 4) {
+            // vmcnt(8): stages s+2, s+3 may be in flight
+            if constexpr (TAIL <= 1) __builtin_amdgcn_s_waitcnt(0x0F78);
+            else if constexpr (TAIL == 2) __builtin_amdgcn_s_waitcnt(0x0F74);
+            else __builtin_amdgcn_s_waitcnt(0x0F70);
+            lds_barrier();
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (TAIL == 0) dma(S, (s + 4) * BK);
+            read_ops((S + 1) & 3, 0, 0);
+        }
+        mfma4(1);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, 1>;
+    using I2 = std::integral_constant<int, 2>;
+    using I3 = std::integral_constant<int, 3>;
+    using I4 = std::integral_constant<int, 4>;
+
+#pragma unroll
+    for (int st = 0; st < 4; ++st) dma(st, st * BK);
+    __builtin_amdgcn_s_waitcnt(0x0F7C);   // vmcnt(12): stage 0 has landed
+    lds_barrier();
+    read_ops(0, 0, 0);
+    // nstages % 4 == 0, so the body is straight-line; the last four stages
+    // are peeled: they request nothing, and every DMA has landed when the
+    // last one starts.
+    for (uint32_t s = 0; s + 4 < nstages; s += 4) {
+        stage(I0{}, I0{}, s);
+        stage(I1{}, I0{}, s + 1);
+        stage(I2{}, I0{}, s + 2);
+        stage(I3{}, I0{}, s + 3);
+    }
+    stage(I0{}, I1{}, nstages - 4);
+    stage(I1{}, I2{}, nstages - 3);
+    stage(I2{}, I3{}, nstages - 2);
+    stage(I3{}, I4{}, nstages - 1);
+    __syncthreads();
+
+    // The two K halves of each 32 x 32 block finish half of it each.  In the
+    // 32x32 accumulator layout (lane l, register r -> row 8 (r / 4) +
+    // 4 (l / 32) + r % 4, column l % 32) registers 0-7 hold rows 0-15 and
+    // registers 8-15 rows 16-31: the wk = 0 wave keeps 0-7 and hands 8-15 to
+    // its partner through LDS, the wk = 1 wave keeps 8-15 and hands 0-7.
+    // Each adds the partner's partial to its own (a + b == b + a exactly, so
+    // the sum does not depend on which wave adds) and stores its 16 rows; C
+    // is written once and not read here: non-temporal stores.
+    float* red = &L[0][0];
+    float* mine = red + ((wave & 3) * 2 + wk) * 8 * 64;
+    const float* theirs = red + ((wave & 3) * 2 + (wk ^ 1)) * 8 * 64;
+    if (wk == 0) {
+#pragma unroll
+        for (int r = 0; r < 8; ++r) mine[r * 64 + lane] = acc[8 + r];
+    } else {
+#pragma unroll
+        for (int r = 0; r < 8; ++r) mine[r * 64 + lane] = acc[r];
+    }
+    __syncthreads();
+    const uint32_t gc = n0 + wn * 32 + li;
+    auto finish = [&](auto base_c) {
+        constexpr int R0 = decltype(base_c)::value;
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+            const float v = acc[R0 + r] + theirs[r * 64 + lane];
+            const uint32_t lr = wm * 32 + 8 * ((R0 + r) >> 2) + 4 * lh + (r & 3);
+            __builtin_nontemporal_store(v, &C[(size_t)(m0 + lr) * g.ldc + gc]);
+        }
+    };
+    if (wk == 0) finish(std::integral_constant<int, 0>{});
+    else finish(std::integral_constant<int, 8>{});
+}
+
 // Small problems (fewer 64 x 64 tiles than half the CUs, K <= 512: the
 // fused_qkv_projection and swiglu registry shapes, the prefill layer's and
 // llama_attention's projections).  There a 64 x 64 tile per workgroup leaves
@@ -395,8 +570,9 @@ void gemm_f32_split_kernel(GemmF32Args g) {
     });
 }
 
+// `f32`: on fp32 MFMA where gemm_f32_dma_kernel takes the shape.
 template <int BL, int EPI, bool RMS>
-int launch_variant(const GemmF32Args& g, uint32_t batch, hipStream_t s) {
+int launch_variant(const GemmF32Args& g, uint32_t batch, hipStream_t s, bool f32 = false) {
     const uint64_t nblocks = (uint64_t)cdiv(g.m, BM) * g.tiles_n;
     if (nblocks > 0x7fffffffull || batch > 65535)
         return fail(MB_E_ARG, "matmul_f32: shape too large");
@@ -415,6 +591,11 @@ int launch_variant(const GemmF32Args& g, uint32_t batch, hipStream_t s) {
         const uint32_t tn32 = cdiv(g.n, 32);
         const dim3 sgrid(cdiv(g.m, 32) * tn32, batch), sblock(64 * cdiv(g.k, 32));
         hipLaunchKernelGGL((gemm_f32_small_kernel<BL, EPI, RMS>), sgrid, sblock, 0, s, g, tn32);
+        MB_LAUNCH_CHECK("matmul_f32");
+        return MB_OK;
+    }
+    if (f32 && vec && g.m % BM == 0 && g.n % BN == 0 && g.k % (4 * BK) == 0 && g.k >= 8 * BK) {
+        hipLaunchKernelGGL(gemm_f32_dma_kernel, dim3((uint32_t)nblocks, batch), dim3(512), 0, s, g);
         MB_LAUNCH_CHECK("matmul_f32");
         return MB_OK;
     }
@@ -456,6 +637,7 @@ int launch_gemm_f32_ex(GemmF32Args g, GemmF32Kind kind, uint32_t batch, hipStrea
     g.tiles_n = cdiv(g.n, BN);
     switch (kind) {
         case GEMM_F32_PLAIN: return launch_variant<BL_KN, EPI_STORE, false>(g, batch, s);
+        case GEMM_F32_PLAIN_MFMA: return launch_variant<BL_KN, EPI_STORE, false>(g, batch, s, true);
         case GEMM_F32_RMS: return launch_variant<BL_KN, EPI_STORE, true>(g, batch, s);
         case GEMM_F32_RMS_BT: return launch_variant<BL_NK, EPI_STORE, true>(g, batch, s);
         case GEMM_F32_RESID: return launch_variant<BL_KN, EPI_RESID, false>(g, batch, s);
@@ -472,9 +654,9 @@ int launch_gemm_f32(const float* a, const float* b, float* c, uint32_t m, uint32
     return launch_gemm_f32_ex(gemm_f32_args(a, b, c, m, n, k), GEMM_F32_PLAIN, 1, s);
 }
 
-// Registry launcher: A@0, B@1 (inputs f32), C@2 (output f32), M@3, N@4, K@5.
-// Also fused_qkv_projection (x @ W_qkv, the same bindings).
-int run_gemm_f32(const Bindings& bs, hipStream_t s, PartMarks*) {
+// Registry launchers: A@0, B@1 (inputs f32), C@2 (output f32), M@3, N@4, K@5.
+// run_gemm_f32 also serves fused_qkv_projection (x @ W_qkv, the same bindings).
+int run_mm(const Bindings& bs, hipStream_t s, GemmF32Kind kind) {
     uint32_t m, n, k;
     int rc;
     if ((rc = bs.u32(3, &m, "M")) || (rc = bs.u32(4, &n, "N")) || (rc = bs.u32(5, &k, "K")))
@@ -484,8 +666,14 @@ int run_gemm_f32(const Bindings& bs, hipStream_t s, PartMarks*) {
         (rc = bs.buffer(1, MB_DTYPE_F32, (uint64_t)k * n * 4, false, &b, "B")) ||
         (rc = bs.buffer(2, MB_DTYPE_F32, (uint64_t)m * n * 4, true, &c, "C")))
         return rc;
-    return launch_gemm_f32((const float*)a, (const float*)b, (float*)c, m, n, k, s);
+    return launch_gemm_f32_ex(gemm_f32_args((const float*)a, (const float*)b, (float*)c, m, n, k), kind, 1, s);
 }
+int run_gemm_f32(const Bindings& bs, hipStream_t s, PartMarks*) { return run_mm(bs, s, GEMM_F32_PLAIN); }
+// sqr_mm is the registry's measure of the fp32 matrix cores: its report is a fraction
+// of their peak, and its profile counts their cycles (one per 64 flop and SIMD, 2^25 at
+// 1024^3).  So this entry stays on fp32 MFMA (1024^3 17.8 us); the same product from
+// mb_launch_matmul_f32 runs in bf16 terms (14.6 us).
+int run_sqr_mm(const Bindings& bs, hipStream_t s, PartMarks*) { return run_mm(bs, s, GEMM_F32_PLAIN_MFMA); }
 
 // batch_mm: A@0 [batch][M][K], B@1 [batch][K][N], C@2 [batch][M][N], M@3, N@4,
 // K@5.  The registry carries no batch scalar (the reference derives it from
@@ -556,11 +744,11 @@ int run_swiglu(const Bindings& bs, hipStream_t s, PartMarks*) {
 void register_gemm_f32() {
     // sqr_mm, rect_mm and fused_qkv_projection share the plain GEMM's spec;
     // the attributes (LDS size, threads) the report prints are those of the
-    // kernel each registry shape runs: the split kernel, or the small-problem
-    // kernel for fused_qkv_projection and swiglu.
+    // kernel each registry shape runs: the split kernel, the DMA kernel for
+    // sqr_mm, or the small-problem kernel for fused_qkv_projection and swiglu.
     const void* plain = reinterpret_cast<const void*>(
         &gemm_f32_split_kernel<BL_KN, EPI_STORE, false>);
-    register_kernel({"sqr_matmul_f32", run_gemm_f32, plain, 1});
+    register_kernel({"sqr_matmul_f32", run_sqr_mm, reinterpret_cast<const void*>(&gemm_f32_dma_kernel), 1});
     register_kernel({"rect_matmul_f32", run_gemm_f32, plain, 1});
     register_kernel({"fused_qkv_projection_f32", run_gemm_f32,
                      reinterpret_cast<const void*>(&gemm_f32_small_kernel<BL_KN, EPI_STORE, false>),

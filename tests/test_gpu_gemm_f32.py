@@ -7,7 +7,7 @@ import pytest
 import torch
 
 import oracle
-from gpu_util import assert_close, launch, ptr, run_registry, seeded
+from gpu_util import assert_close, launch, ptr, run_bound, run_registry, seeded
 
 pytestmark = pytest.mark.gpu
 
@@ -201,3 +201,15 @@ def test_matmul_f32_very_wide_rows(mb, dev, dual):
     assert torch.isinf(c[0, at])
     c[0, at] = want
     assert (c - want).abs().max().item() <= 1e-6 * want
+
+
+# sqr_mm's kernel (fp32 MFMA fed by DMA: full tiles, K a multiple of 256 from 512): the
+# shortest K that reaches it, two and more trips of its loop, one tile and many
+@pytest.mark.parametrize("m,n,k", [(1024, 512, 512), (64, 64, 768), (192, 128, 1024), (576, 640, 1280)])
+def test_sqr_mm_full_tiles(mb, m, n, k):
+    a, b = seeded(m + k, (m, k)), seeded(n + k, (k, n))
+    (c,) = run_bound("sqr_matmul_f32", [(0, a), (1, b)], [(2, (m, n))],
+                     [(3, "u32", m), (4, "u32", n), (5, "u32", k)])
+    A, B = a.numpy().astype(np.float64), b.numpy().astype(np.float64)
+    # a chain of k / 2 roundings to 2^-24 of a partial sum per K half, random in sign
+    assert np.all(np.abs(c.numpy() - A @ B) <= 2.0 ** -20 * (np.abs(A) @ np.abs(B)))

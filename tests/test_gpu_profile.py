@@ -40,18 +40,16 @@ def _samples(out: str) -> dict:
 
 
 def test_profile_sqr_mm_mfma_busy_cycles_closed_form():
-    """The 1024^3 GEMM multiplies on bf16 MFMAs, six term products to one fp32
-    product (h h, h m, m h, m m, h l, l h).  Every 32x32x16 bf16 MFMA retires
-    1024 flop per SIMD-cycle, so 6 x 2^31 flop keep the MFMA pipe busy for
-    exactly 6 x 2^31 / 1024 = 6 x 2^21 cycles, whatever the tile shape (1024
-    is a multiple of every tile, so no MFMA works on padding).  On fp32 MFMAs
-    (64 flop per SIMD-cycle) it would be 2^25."""
+    """Every fp32 MFMA retires 64 flop per SIMD-cycle (256 per CU-clock), so
+    the 1024^3 GEMM's 2^31 flop keep the MFMA pipe busy for exactly
+    2^31 / 64 = 2^25 cycles, whatever the tile shape (1024 is a multiple of
+    every tile, so no MFMA works on padding)."""
     r, out = _bench("sqr_mm", "--no-save", "--", "--no-session", "--profile",
                     "--iters", "5", "--warmup", "2", "--cpu-iters", "1")
     assert r.returncode == 0, out[-3000:]
     assert "correctness : ✓" in out
     s = _samples(out)
-    assert s["SQ_VALU_MFMA_BUSY_CYCLES"] == 6 * 2 ** 21, s
+    assert s["SQ_VALU_MFMA_BUSY_CYCLES"] == 2 ** 25, s
     assert s["SQ_INSTS_MFMA"] > 0 and s["GRBM_GUI_ACTIVE"] > 0
     # the counter-set line lists what the passes sample
     assert re.search(r"^  counters    : GRBM_GUI_ACTIVE, .*WRITE_SIZE$", out, re.M), out[-3000:]
