@@ -41,8 +41,8 @@ constexpr int KQ = BK / 4;     // float4s per K-contiguous row of a stage
 constexpr int SA = BK + 4;   // As (and transposed Bs) row stride (floats)
 constexpr int SB = BN + 4;   // Bs row stride (floats)
 
-// Operands of 2 GB or more, which 32-bit buffer offsets do not reach (and K =
-// 0): fp32 MFMA, element-wise guarded loads through 64-bit addresses.
+// Operands of 2 GB or more and C rows of more than 8 million columns, which 32-bit buffer
+// offsets do not reach (and K = 0): fp32 MFMA, element-wise guarded loads through 64-bit addresses.
 //  * BK = 64 per stage, LDS double buffered, one barrier per stage; operands
 //    are register-staged two stages ahead;
 //  * 4 waves own a 2x2 grid of 32x32 sub-tiles (v_mfma_f32_32x32x2f32);
@@ -600,8 +600,13 @@ int launch_variant(const GemmF32Args& g, uint32_t batch, hipStream_t s, bool f32
         return MB_OK;
     }
     // every other shape, at any alignment: bf16 term products, unless 32-bit
-    // buffer offsets do not reach an operand (2 GB) or K is 0
-    const uint64_t c_bytes = (uint64_t)g.m * std::max(g.ldc, g.ldr) * 4;
+    // buffer offsets do not reach an operand or a tile's 64 rows of C (2 GB), or K
+    // is 0.  (C itself may be larger: 32768 x 16384 x 1024 6540 us, 8440 on fp32 MFMA, 16550
+    // with the element-wise loads below.)  Short K and many tiles, which leave some
+    // of the waves without a unit, are faster here too: 2048 x 2048 x 16 10.8 us against
+    // 17.1 for register-staged fp32 MFMA tiles, x 64 12.8 and 16.9, 4096 x 4096 x 32 35.4
+    // and 56.6, 100 x 60000 x 64 20.8 and 28.7.
+    const uint64_t c_bytes = (uint64_t)std::min(g.m, 64u) * std::max(g.ldc, g.ldr) * 4;
     if (g.k > 0 && (uint64_t)g.m * g.lda * 4 < 0x80000000ull && b_rows * g.ldb * 4 < 0x80000000ull &&
         c_bytes < 0x80000000ull) {
         GemmF32Args q = g;

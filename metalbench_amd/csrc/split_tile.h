@@ -307,8 +307,11 @@ __device__ __forceinline__ void split_tile(const SplitTile& g, DmaA dma_a) {
             return __builtin_amdgcn_make_buffer_rsrc(
                 const_cast<float*>(p), 0, __builtin_amdgcn_readfirstlane(bytes), 0x00020000u);
         };
-        const __amdgpu_buffer_rsrc_t crs = rsrc(C, extent(M, g.ldc, N));
-        const __amdgpu_buffer_rsrc_t rrs = EPI == EPI_RESID ? rsrc(g.r, extent(M, g.ldr, N)) : crs;
+        // (from the tile's first row, so that C and R may pass 4 GB)
+        const uint32_t rows = min(M - m0, 64u);
+        const __amdgpu_buffer_rsrc_t crs = rsrc(C + (size_t)m0 * g.ldc, extent(rows, g.ldc, N));
+        const __amdgpu_buffer_rsrc_t rrs =
+            EPI == EPI_RESID ? rsrc(g.r + (size_t)m0 * g.ldr, extent(rows, g.ldr, N)) : crs;
 #pragma unroll
         for (int q = 0; q < QN; ++q) {
             const uint32_t lr = 32 * i + 8 * ((q0 + q) >> 2) + 4 * lh + (q & 3), gr = m0 + lr;
@@ -327,9 +330,9 @@ __device__ __forceinline__ void split_tile(const SplitTile& g, DmaA dma_a) {
                 if (DUAL) out = silu_f(out) * (v[1][q] * sc);
                 if (EPI == EPI_RESID)
                     out += __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-                        rrs, in ? (gr * g.ldr + gc) * 4 : 0x80000000u, 0, 0));
+                        rrs, in ? (lr * g.ldr + gc) * 4 : 0x80000000u, 0, 0));
                 __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(out), crs,
-                                                      in ? (gr * g.ldc + gc) * 4 : 0x80000000u, 0, 0);
+                                                      in ? (lr * g.ldc + gc) * 4 : 0x80000000u, 0, 0);
             }
         }
         return false;

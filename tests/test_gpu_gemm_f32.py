@@ -213,3 +213,22 @@ def test_sqr_mm_full_tiles(mb, m, n, k):
     A, B = a.numpy().astype(np.float64), b.numpy().astype(np.float64)
     # a chain of k / 2 roundings to 2^-24 of a partial sum per K half, random in sign
     assert np.all(np.abs(c.numpy() - A @ B) <= 2.0 ** -20 * (np.abs(A) @ np.abs(B)))
+
+
+@pytest.mark.parametrize("m,n,k", [(40000, 16001, 130), (100, 6_000_000, 5), (70, 9_000_000, 4)])
+def test_matmul_f32_output_past_2gb(mb, dev, m, n, k):
+    """C past 2 GB from small operands; the last shape's rows pass what a tile's 32-bit
+    offsets reach."""
+    gen = torch.Generator(device=dev).manual_seed(5)
+    a = torch.empty((m, k), device=dev).uniform_(-1, 1, generator=gen)
+    b = torch.empty((k, n), device=dev).uniform_(-1, 1, generator=gen)
+    buf = torch.full((m * n + 64,), 7.0, device=dev)
+    launch("mb_launch_matmul_f32", ptr(a), ptr(b), ptr(buf), m, n, k, None)
+    c = buf[:m * n].view(m, n)
+    for rows in range(0, m, 4000):
+        A, B = a[rows:rows + 4000].double(), b.double()
+        for cols in range(0, n, 1_000_000):
+            Bc = B[:, cols:cols + 1_000_000]
+            off = (c[rows:rows + 4000, cols:cols + 1_000_000] - A @ Bc).abs()
+            assert (off <= 2.0 ** -22 * (A.abs() @ Bc.abs())).all(), (rows, cols)
+    assert (buf[m * n:] == 7.0).all()
