@@ -22,8 +22,8 @@
 //    tile leaves CUs idle below 256 tiles, and unaligned rows were loaded element
 //    by element: 1000 x 3000 x 4096 159 -> 36 us, 1001 x 3001 x 4095 457 -> 71,
 //    128 x 4096 x 4096 148 -> 15, 64 x 512 x 4096 142 -> 7.4;
-//  * operands or results past 2 GB that are not full tiles, more than 16 million
-//    columns with K < 128, and K = 0 take
+//  * operands or results past 2 GB that are not full tiles, a C off a 4-byte boundary
+//    likewise, more than 16 million columns with K < 128, and K = 0 take
 //    gemm_bf16_kernel (4 x 4 v_mfma_f32_32x32x16_bf16 per wave), BK = 64 with an LDS
 //    double buffer:
 //    both operands stored K-contiguous, row pitch 72 bf16 (144 B), 2 x 2 x
@@ -266,6 +266,7 @@ typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4_t;
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef u32x4 u32x4_any __attribute__((aligned(2)));   // 16 bytes at any element of C: one store instruction all the same
 template <int V> struct TailC { static constexpr int v = V; };
 
 // EDGE: M and N of any size (N even), K a multiple of 8: rows past M read row M - 1,
@@ -552,7 +553,7 @@ void gemm_bf16_full_kernel(const uint16_t* __restrict__ A, const uint16_t* __res
         const uint32_t gr = m0 + wm * 128 + row, gc = n0 + wn * 128 + 8 * ch;
         uint16_t* at = C + (size_t)gr * N + gc;
         if (!EDGE || ((N & 7) == 0 && ((uintptr_t)C & 15) == 0)) {
-            if (!EDGE || (gr < M && gc < N)) __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(at));
+            if (!EDGE || (gr < M && gc < N)) __builtin_nontemporal_store(v, reinterpret_cast<u32x4_any*>(at));
         } else if (gr < M) {
 #pragma unroll
             for (int e = 0; e < 8; ++e)
@@ -1232,20 +1233,22 @@ int launch_gemm_bf16(const uint16_t* a, const uint16_t* b, uint16_t* c, uint32_t
     const bool near = k > 0 && (uint64_t)m * k * 2 < (1ull << 31) && (uint64_t)k * n * 2 < (1ull << 31) &&
                       (uint64_t)m * n * 2 < (1ull << 31) &&
                       (((uint64_t)k + 127) & ~127ull) * n * 2 < (1ull << 32);
-    // Full 256 x 256 tiles, more than 64 of them (or a C past 2 GB).  Up to 64, one
-    // round of tiles a quarter as large or smaller is faster (512 x 6144 x 4096: 66
-    // us on 48 tiles, 36 on 256; 2048^3: 37 and 22); from 65 it takes two rounds (2048 x
-    // 4096 x 1024: 23 us and 25).
+    const bool tiles = near && (((uintptr_t)c) & 3) == 0;   // (the k-wave kernel stores dwords)
+    // Full 256 x 256 tiles, more than 64 of them (or a C past 2 GB, or off a 4-byte
+    // boundary).  Up to 64, one round of tiles a quarter as large or smaller is faster
+    // (512 x 6144 x 4096: 66 us on 48 tiles, 36 on 256; 2048^3: 37 and 22); from 65 it
+    // takes two rounds (2048 x 4096 x 1024: 23 us and 25).  C may lie anywhere: 4096^3
+    // with C 4 or 2 bytes off 94 us (guarded tiles, which store elements, 113;
+    // gemm_bf16_kernel 164).
     const bool full = aligned && m % BM == 0 && n % BN == 0 && k % (2 * BK) == 0 && k > 0 &&
-                      (uint64_t)m * k * 2 < (1ull << 31) && (uint64_t)k * n * 2 < (1ull << 31) &&
-                      (((uintptr_t)c) & 15) == 0;
-    if (full && (nblocks > 64 || !near)) {
+                      (uint64_t)m * k * 2 < (1ull << 31) && (uint64_t)k * n * 2 < (1ull << 31);
+    if (full && (nblocks > 64 || !tiles)) {
         hipLaunchKernelGGL(gemm_bf16_full_kernel<false>, dim3((uint32_t)nblocks), dim3(256), 0, s, a, b, c,
                            m, n, k, tiles_m, tiles_n);
         MB_LAUNCH_CHECK("matmul_bf16");
         return MB_OK;
     }
-    if (near && (((uintptr_t)c) & 3) == 0) return launch_tiles(a, b, c, m, n, k, s);
+    if (tiles) return launch_tiles(a, b, c, m, n, k, s);
     static bool attr_set[3] = {false, false, false};
     auto go = [&](auto kernel, int mode) -> int {
         if (!attr_set[mode]) {

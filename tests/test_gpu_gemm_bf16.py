@@ -169,3 +169,21 @@ def test_matmul_bf16_very_wide_rows(mb, dev):
     assert torch.isinf(c[0, at])
     c[0, at] = 2.0
     assert (c == 2.0).all()
+
+
+@pytest.mark.parametrize("m,n,k", [(2304, 2048, 128), (256, 512, 256)])
+@pytest.mark.parametrize("shift", [1, 2, 4])
+def test_matmul_bf16_full_tiles_into_unaligned_c(mb, dev, m, n, k, shift):
+    """Full tiles, more and fewer than 64, with C off a 16-byte boundary."""
+    a = seeded(m + k, (m, k), ("normal", 0.0, 1.0), "bf16").to(dev)
+    b = seeded(n + k, (k, n), ("normal", 0.0, 1.0), "bf16").to(dev)
+    buf = torch.full((m * n + 16,), 7.0, dtype=torch.bfloat16, device=dev)
+    launch("mb_launch_matmul_bf16", ptr(a), ptr(b), buf.data_ptr() + 2 * shift, m, n, k, None)
+    c = torch.full((m, n), 7.0, dtype=torch.bfloat16, device=dev)
+    launch("mb_launch_matmul_bf16", ptr(a), ptr(b), ptr(c), m, n, k, None)
+    got = buf.float().cpu().numpy()
+    assert np.all(got[:shift] == 7.0) and np.all(got[shift + m * n:] == 7.0)
+    A, B = oracle.as_f64(a), oracle.as_f64(b)
+    want, size = A @ B, np.abs(A) @ np.abs(B)
+    for x in (got[shift:shift + m * n].reshape(m, n), c.float().cpu().numpy()):
+        assert np.all(np.abs(x - want) <= 2.0 ** -8 * np.abs(want) + 2.0 ** -20 * size)
