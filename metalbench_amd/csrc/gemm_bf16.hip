@@ -1186,18 +1186,23 @@ int launch_wave_tile(const uint16_t* a, const uint16_t* b, uint16_t* c, uint32_t
     return MB_OK;
 }
 
-int launch_tiles(const uint16_t* a, const uint16_t* b, uint16_t* c, uint32_t m, uint32_t n,
-                 uint32_t k, hipStream_t s) {
-    const bool odd = ((k | n) & 1) || ((((uintptr_t)a) | ((uintptr_t)b)) & 3);
+// The cheapest tile, or nullptr: none can be launched.
+const TileChoice* choose_tile(uint32_t m, uint32_t n, uint32_t k, bool odd) {
     const TileChoice* best = nullptr;
     float least = 0.f;
     for (const TileChoice& t : k_tiles) {
         if (odd ? t.odd_c1 == 0.f : t.kind == TILE_EDGE && k % 8) continue;
         const uint64_t tiles = (uint64_t)cdiv(m, t.tm) * cdiv(n, t.tn);
+        if (tiles >= 1u << 23) continue;   // 2^32 threads or more (512 to a tile) cannot be launched
         const float cost = (float)((tiles + 255) / 256) *
                            (odd ? t.odd_c0 + t.odd_c1 * cdiv(k, 32) : t.c0 + t.c1 * cdiv(k, 32));
         if (!best || cost < least) { best = &t; least = cost; }
     }
+    return best;
+}
+
+int launch_tiles(const TileChoice* best, const uint16_t* a, const uint16_t* b, uint16_t* c, uint32_t m,
+                 uint32_t n, uint32_t k, bool odd, hipStream_t s) {
     if (best->kind == TILE_EDGE) {
         const uint32_t tm = cdiv(m, BM), tn = cdiv(n, BN);
         hipLaunchKernelGGL(gemm_bf16_full_kernel<true>, dim3(tm * tn), dim3(256), 0, s, a, b, c, m, n, k,
@@ -1248,7 +1253,10 @@ int launch_gemm_bf16(const uint16_t* a, const uint16_t* b, uint16_t* c, uint32_t
         MB_LAUNCH_CHECK("matmul_bf16");
         return MB_OK;
     }
-    if (tiles) return launch_tiles(a, b, c, m, n, k, s);
+    if (tiles) {
+        const bool odd = ((k | n) & 1) || ((((uintptr_t)a) | ((uintptr_t)b)) & 3);
+        if (const TileChoice* t = choose_tile(m, n, k, odd)) return launch_tiles(t, a, b, c, m, n, k, odd, s);
+    }
     static bool attr_set[3] = {false, false, false};
     auto go = [&](auto kernel, int mode) -> int {
         if (!attr_set[mode]) {

@@ -187,3 +187,15 @@ def test_matmul_bf16_full_tiles_into_unaligned_c(mb, dev, m, n, k, shift):
     want, size = A @ B, np.abs(A) @ np.abs(B)
     for x in (got[shift:shift + m * n].reshape(m, n), c.float().cpu().numpy()):
         assert np.all(np.abs(x - want) <= 2.0 ** -8 * np.abs(want) + 2.0 ** -20 * size)
+
+
+def test_matmul_bf16_more_rows_than_small_tiles_can_launch(mb, dev):
+    """2^30 - 1 rows of one odd-shaped element: 2^24 tiles of 64 rows would be 2^32
+    threads, one more than a launch may have."""
+    m = 2 ** 30 - 1
+    a = torch.arange(m, device=dev, dtype=torch.int32).remainder_(251).to(torch.bfloat16)
+    b = torch.full((1,), 2.0, device=dev, dtype=torch.bfloat16)
+    c = torch.zeros((m,), device=dev, dtype=torch.bfloat16)
+    launch("mb_launch_matmul_bf16", ptr(a), ptr(b), ptr(c), m, 1, 1, None)
+    for at in range(0, m, 2 ** 28):
+        assert torch.equal(c[at:at + 2 ** 28], a[at:at + 2 ** 28] * 2.0)
