@@ -45,6 +45,7 @@
 #include "common.h"
 
 #include <algorithm>
+#include <atomic>
 #include <type_traits>
 
 namespace mb {
@@ -1163,9 +1164,12 @@ int launch_grid_tile(const uint16_t* a, const uint16_t* b, uint16_t* c, uint32_t
     constexpr uint32_t ring = R * KG * (32 * MB + 32 * NB) * 64 + 1024, sums = KG == 2 ? 4096 * MB * NB : 0;
     constexpr uint32_t lds = ring > sums ? ring : sums;
     const auto kernel = gemm_bf16_tile_kernel<MB, NB, KG, R, ODD>;
-    static const hipError_t attr = hipFuncSetAttribute(
-        reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    MB_HIP_TRY(attr);
+    static std::atomic<bool> ready{false};   // (a failure is not kept: the next call tries again)
+    if (!ready.load(std::memory_order_acquire)) {
+        MB_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        ready.store(true, std::memory_order_release);
+    }
     hipLaunchKernelGGL(kernel, dim3(tm * tn), dim3(256 * KG), lds, s, a, b, c, m, n, k, tm, tn,
                        std::min(tm, (uint32_t)GM));
     MB_LAUNCH_CHECK("matmul_bf16");
