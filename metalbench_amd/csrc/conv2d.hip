@@ -38,7 +38,9 @@ constexpr int BM = 64, BN = 64, BK = 32;
 constexpr int SK = BK + 4;   // LDS row stride (floats), both operands
 constexpr int KQ = BK / 4;   // float4s per K-contiguous row of a stage
 
-// x / d for x < 2^31 without a branch: (umulhi(x, mul) + (x & one)) >> sh
+// floor(x / d) for x < 2^31 without a branch, from divisor(d) (launch_conv2d).  (Pixel
+// and k indices stay below 2^31: the kernels that divide by it take M O 4 < 2^31 and
+// O K 4 < 2^31 only.)
 struct Divisor { uint32_t mul, sh, one; };   // one = all bits for d = 1 (mul 0)
 __device__ __forceinline__ uint32_t div_any(uint32_t x, Divisor d) {
     return (__umulhi(x, d.mul) + (x & d.one)) >> d.sh;
@@ -48,16 +50,8 @@ struct ConvShape {
     uint32_t n, h, w, c, o, r, s, stride, pad, p, q;
     uint32_t m;   // n*p*q
     uint32_t k;   // r*s*c
-    uint32_t q_mul, q_sh, p_mul, p_sh;   // x / q and x / p for x < 2^31 (mul 0: divisor 1)
-    Divisor dq, dp, dc, ds;              // x / q, x / p, x / c, x / s (div_any)
+    Divisor dq, dp, dc, ds;              // x / q, x / p, x / c, x / s
 };
-
-// floor(x / d) for x < 2^31 from (mul, sh) = magic_u31(d) (launch_conv2d).
-// The DMA kernel divides pixel indices below M, and its path requires
-// M O 4 < 2^31.
-__device__ __forceinline__ uint32_t div_magic(uint32_t x, uint32_t mul, uint32_t sh) {
-    return mul ? __umulhi(x, mul) >> sh : x;
-}
 
 template <int KSPLIT>
 __global__ __launch_bounds__(256 * KSPLIT)
@@ -281,8 +275,8 @@ void conv2d_f32_dma_kernel(const float* __restrict__ X, const float* __restrict_
     const uint32_t mm = m_ok ? m : 0;
     // (multiply-high divisions: the compiler's 32-bit divide is ~20 VALU
     // instructions, and this set-up runs beside other workgroups' MFMA loops)
-    const uint32_t t = div_magic(mm, sh.q_mul, sh.q_sh), qq = mm - t * sh.q;
-    const uint32_t nn = div_magic(t, sh.p_mul, sh.p_sh), pp = t - nn * sh.p;
+    const uint32_t t = div_any(mm, sh.dq), qq = mm - t * sh.q;
+    const uint32_t nn = div_any(t, sh.dp), pp = t - nn * sh.p;
     const int32_t h0 = (int32_t)(pp * sh.stride) - (int32_t)sh.pad;
     const int32_t w0 = (int32_t)(qq * sh.stride) - (int32_t)sh.pad;
     const uint32_t xbase = (nn * sh.h * sh.w * sh.c + 4 * dch) * 4;   // bytes
@@ -540,20 +534,12 @@ int launch_conv2d(const float* x, const float* w, float* y, uint32_t n, uint32_t
     // floor(x / d) = umulhi(x, M) >> (s - 1) for x < 2^31, with s = ceil(log2 d)
     // and M = floor(2^(31+s) / d) + 1 < 2^32: M d - 2^(31+s) lies in (0, d],
     // so x (M d - 2^(31+s)) < 2^31 d <= 2^(31+s) and the error stays below
-    // one step.  d = 1 takes the plain path (mul 0).
-    auto magic_u31 = [](uint32_t d, uint32_t* mul, uint32_t* shift) {
-        if (d <= 1) { *mul = 0; *shift = 0; return; }
+    // one step.  d = 1 (or 0, of an empty shape) gives x itself.
+    auto divisor = [](uint32_t d) {
+        if (d <= 1) return Divisor{0, 0, ~0u};
         uint32_t l = 0;
         while ((1ull << l) < d) ++l;
-        *mul = (uint32_t)(((1ull << (31 + l)) / d) + 1);
-        *shift = l - 1;
-    };
-    magic_u31(sh.q, &sh.q_mul, &sh.q_sh);
-    magic_u31(sh.p, &sh.p_mul, &sh.p_sh);
-    auto divisor = [&](uint32_t d) {
-        Divisor v{0, 0, d <= 1 ? ~0u : 0u};
-        magic_u31(d, &v.mul, &v.sh);
-        return v;
+        return Divisor{(uint32_t)(((1ull << (31 + l)) / d) + 1), l - 1, 0};
     };
     sh.dq = divisor(sh.q);
     sh.dp = divisor(sh.p);

@@ -748,7 +748,6 @@ void gemm_bf16_tile_kernel(const uint16_t* __restrict__ A, const uint16_t* __res
     // at most `younger` stages' DMAs of this wave still in flight
     auto wait = [&](uint32_t younger) {
         if (younger >= R - 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((R - 2) * NW) : "memory");
-        else if (R > 6 && younger >= 4) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 * NW) : "memory");
         else if (younger >= 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NW) : "memory");
         else if (younger == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NW) : "memory");
         else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");

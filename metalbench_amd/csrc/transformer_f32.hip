@@ -688,7 +688,6 @@ int run_llama_attention(const Bindings& bs, hipStream_t s, PartMarks*) {
     if ((rc = launch_gemm_f32_ex(gemm_f32_args((const float*)x, (const float*)wqkv, qkv, S, nqkv, D),
                                  GEMM_F32_PLAIN, 1, s)))
         return rc;
-    if (S == 0) return MB_OK;
     AttnPrefillArgs<float> a{qkv, attn, S, D, H, HKV, nqkv, D, 1.0f / sqrtf((float)dh), (double)base};
     if ((uint64_t)S * (dh / 2) <= ROT_PAIRS) {
         if ((rc = launch_attention_prefill<float, true>(a, dh, s))) return rc;
