@@ -77,3 +77,40 @@ def run_bound(metal_function: str, inputs, outputs, scalars, dtype="f32"):
     native.run(native.kernel_find(metal_function), binds, 0, 1, native.RUN_SYNC_EACH)
     sync()
     return [t.cpu() for _, t in d_out]
+
+
+# bf16 products by the tile that takes them: (kind, mb, nb) as in gemm_bf16.hip's k_tiles,
+# the tile for even K and N, the tile where K or N is odd or A or B lies off a 4-byte
+# boundary.  One past or one short of a tile in M and N, and K of a single short stage,
+# a few stages with a remainder, and many.
+BF16_TILE_SHAPES = [
+    ((1537, 4610, 8), ("EDGE", 0, 0), ("GRID", 4, 4)),
+    ((1537, 4610, 392), ("EDGE", 0, 0), ("GRID", 4, 4)),
+    ((513, 3586, 2), ("GRID", 8, 4), ("GRID", 4, 3)),
+    ((769, 4610, 290), ("GRID", 8, 4), ("WAVE", 4, 8)),
+    ((513, 4990, 130), ("GRID", 4, 4), ("GRID", 4, 4)),
+    ((513, 4990, 290), ("GRID", 4, 4), ("GRID", 4, 4)),
+    ((513, 4990, 514), ("GRID", 4, 4), ("GRID", 4, 4)),
+    ((513, 4990, 1), None, ("GRID", 4, 4)),
+    ((513, 4990, 289), None, ("GRID", 4, 4)),
+    ((385, 4702, 130), ("GRID", 4, 3), ("GRID", 4, 3)),
+    ((385, 4702, 514), ("GRID", 4, 3), ("GRID", 4, 3)),
+    ((385, 4702, 1), None, ("GRID", 4, 3)),
+    ((385, 4701, 513), None, ("GRID", 4, 3)),
+    ((2367, 386, 2), ("WAVE", 4, 8), ("WAVE", 4, 8)),
+    ((193, 4098, 1026), ("WAVE", 4, 8), ("WAVE", 2, 4)),
+    ((2367, 385, 1), None, ("WAVE", 4, 8)),
+    ((2367, 385, 1025), None, ("WAVE", 4, 8)),
+    ((2049, 194, 2), ("WAVE", 4, 4), ("WAVE", 4, 4)),
+    ((2049, 194, 1026), ("WAVE", 4, 4), ("WAVE", 4, 4)),
+    ((2049, 193, 1025), None, ("WAVE", 4, 4)),
+    ((1025, 194, 2), ("WAVE", 2, 4), ("WAVE", 2, 4)),
+    ((1025, 194, 1026), ("WAVE", 2, 4), ("WAVE", 2, 4)),
+    ((1025, 193, 1025), None, ("WAVE", 2, 4)),
+    ((17, 4098, 2), ("WAVE", 1, 4), ("WAVE", 1, 4)),
+    ((17, 4098, 1026), ("WAVE", 1, 4), ("WAVE", 1, 4)),
+    ((17, 4097, 1025), None, ("WAVE", 1, 4)),
+    ((1, 2, 2), ("WAVE", 1, 2), ("WAVE", 1, 2)),
+    ((33, 66, 1026), ("WAVE", 1, 2), ("WAVE", 1, 2)),
+    ((33, 65, 1025), None, ("WAVE", 1, 2)),
+]

@@ -11,7 +11,7 @@ import pytest
 import torch
 
 import oracle
-from gpu_util import assert_close, launch, ptr, run_registry, seeded
+from gpu_util import BF16_TILE_SHAPES, assert_close, launch, ptr, run_registry, seeded
 from metalbench_amd import native
 
 pytestmark = pytest.mark.gpu
@@ -108,19 +108,21 @@ def test_kernel_attrs_report_register_split(mb):
 # Shapes away from full 256 x 256 tiles: each kind of tile, one past and one short
 # of a tile, of a 32-deep stage and of a chunk of 8, even and odd rows.
 @pytest.mark.parametrize("m,n,k", [
-    (3001, 3002, 136), (2815, 2900, 72),            # guarded 256 x 256 tiles
-    (3000, 3002, 70), (2049, 3970, 250),            # 256 x 128
-    (1025, 2050, 322), (1000, 3000, 98),            # 128 x 128, 128 x 96
-    (1001, 3001, 97), (1023, 2047, 289),            # the same, odd rows
-    (513, 1026, 130), (511, 1023, 131),             # 64 x 128 and 64 x 64
+    (3001, 3002, 136),                              # guarded 256 x 256 tiles
+    (2815, 2900, 72), (3000, 3002, 70), (2049, 3970, 250), (1000, 3000, 98),   # 256 x 128
+    (1025, 2050, 322), (1001, 3001, 97),            # 128 x 96, even and odd rows
+    (1023, 2047, 289),                              # 64 x 128, odd rows
+    (513, 1026, 130), (511, 1023, 131),             # 64 x 64, 32 x 64 odd rows
+    # 16 x 32
     (33, 66, 34), (31, 65, 33), (130, 200, 1026), (129, 199, 1025),
     (17, 34, 2), (15, 33, 1), (16, 30, 4098), (17, 31, 4097),
 ])
 @pytest.mark.parametrize("shift", [0, 1])
 def test_matmul_bf16_tile_edges(mb, dev, m, n, k, shift):
-    """Also from pointers 2 bytes off a 4-byte boundary; nothing is written around C, and
-    an infinite row of A (whose values follow the row before it in memory) reaches only
-    its own outputs."""
+    """Also with all three matrices 2 bytes off a 4-byte boundary (a C there is left to
+    the kernel with 64-bit addresses); nothing is written around C, and an infinite row
+    of A (whose values follow the row before it in memory) reaches only its own
+    outputs."""
     a = seeded(m + k, (m, k), ("normal", 0.0, 1.0), "bf16")
     b = seeded(n + k, (k, n), ("normal", 0.0, 1.0), "bf16")
     bad = m // 2
@@ -199,3 +201,33 @@ def test_matmul_bf16_more_rows_than_small_tiles_can_launch(mb, dev):
     launch("mb_launch_matmul_bf16", ptr(a), ptr(b), ptr(c), m, 1, 1, None)
     for at in range(0, m, 2 ** 28):
         assert torch.equal(c[at:at + 2 ** 28], a[at:at + 2 ** 28] * 2.0)
+
+
+@pytest.mark.parametrize("shape", [s for s, _, _ in BF16_TILE_SHAPES], ids=str)
+@pytest.mark.parametrize("off", ["", "a", "b", "ab", "c"])
+def test_matmul_bf16_every_tile(mb, dev, shape, off):
+    """Every tile, for even and odd rows, with A, B or both 2 bytes off a 4-byte boundary
+    (the tiles for odd rows then take even K and N as well) or C 4 bytes off a 16-byte
+    one.  The infinite row and what surrounds C as in test_matmul_bf16_tile_edges."""
+    m, n, k = shape
+    gen = torch.Generator(device=dev).manual_seed(m + n + k)
+    put = {"a": 0, "b": 0, "c": 2 if off == "c" else 0}
+    put.update({x: 1 for x in off if x in "ab"})
+    buf = {x: torch.full((r * c + 16,), 7.0, dtype=torch.bfloat16, device=dev)
+           for x, r, c in (("a", m, k), ("b", k, n), ("c", m, n))}
+    view = {x: buf[x][put[x]:put[x] + r * c].view(r, c) for x, r, c in (("a", m, k), ("b", k, n), ("c", m, n))}
+    for x in "ab":
+        view[x].copy_(torch.empty(view[x].shape, device=dev).normal_(generator=gen))
+    bad = m // 2 if m > 1 else None
+    if bad is not None:
+        view["a"][bad] = float("inf")
+    launch("mb_launch_matmul_bf16", *[view[x].data_ptr() for x in "abc"], m, n, k, None)
+    rows = torch.ones(m, dtype=torch.bool, device=dev)
+    if bad is not None:
+        rows[bad] = False
+        assert not torch.isfinite(view["c"][bad]).any()
+    A, B = view["a"][rows].double(), view["b"].double()
+    want = A @ B
+    # bf16 rounding (2^-8 of the result) and fp32 sums (2^-20 of the products' magnitudes)
+    assert ((view["c"][rows].double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -20 * (A.abs() @ B.abs())).all()
+    assert (buf["c"][:put["c"]] == 7.0).all() and (buf["c"][put["c"] + m * n:] == 7.0).all()
