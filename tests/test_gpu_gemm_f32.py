@@ -1,4 +1,4 @@
-"""fp32 MFMA GEMM (sqr_mm / rect_mm) on the GPU vs the float64 oracle.
+"""fp32 GEMM (matmul_f32, sqr_mm, rect_mm) on the GPU vs the float64 oracle.
 
 Tolerance: rtol = atol = 1e-4 for the sqr_mm benchmark config, scaled with
 sqrt(K) for the normal(0,1) shapes where |C| grows with K."""
@@ -19,8 +19,8 @@ pytestmark = pytest.mark.gpu
     # (32x32 tiles, K over up to 16 waves): K = 32 (one wave), 464 (15 waves,
     # the last one's slice half past K), ragged M and N
     (32, 96, 32), (96, 64, 464), (70, 130, 256),
-    # full tiles with K % 256 == 0 and K >= 512 (and, at K = 512, at least 128
-    # tiles) take the LDS-DMA kernel: two loop trips, three trips
+    # full tiles and whole 16-deep units on the kernel of bf16 term products, as
+    # every other shape: 8 and 12 units per wave
     (1024, 512, 512), (192, 128, 768),
 ])
 def test_matmul_f32_shapes(mb, dev, m, n, k):
@@ -35,7 +35,7 @@ def test_matmul_f32_shapes(mb, dev, m, n, k):
 
 def _random_f32_shapes(n, seed=72):
     """Seeded shapes: half ragged, half full 64 x 64 tiles with K a multiple of
-    256 from 512 (the LDS-DMA kernel from K = 768, the small-problem kernel at
+    256 from 512 (bf16 term products from K = 768, the small-problem kernel at
     K = 512 when there are fewer than 128 tiles)."""
     rng = np.random.default_rng(seed)
     out = []
@@ -60,7 +60,7 @@ def test_matmul_f32_k0_gives_zeros(mb, dev):
     assert torch.all(d_c.cpu() == 0.0)
 
 
-# small-problem kernel, register-staged kernel (ragged), LDS-DMA kernel
+# small-problem kernel, then bf16 term products: ragged and full tiles
 @pytest.mark.parametrize("n", [192, 1000, 1024])
 def test_matmul_f32_identity_exact(mb, dev, n):
     a = seeded(3, (n, n))

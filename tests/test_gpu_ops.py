@@ -101,7 +101,8 @@ def test_rms_norm_row_widths(mb, rows, cols, add):
 
 
 @pytest.mark.parametrize("m,n,k", [(70, 90, 130), (64, 64, 64), (1, 3, 5),
-                                   # full 64-tiles, K a multiple of 256: the LDS-DMA kernel
+                                   # full 64 x 64 tiles: the small-problem kernel (K = 512),
+                                   # then bf16 term products
                                    (128, 192, 512), (64, 320, 768), (192, 64, 1024)])
 def test_rms_norm_linear_shapes(mb, m, n, k):
     x, w = seeded(4, (m, k)), seeded(5, (n, k))
