@@ -17,8 +17,9 @@
 //    slots of whole 128-byte lines, B in 32-deep slots), B transposed by the
 //    LDS reads (ds_read_b64_tr_b16);
 //  * other shapes take the cheapest of k_tiles: the same kernel with guarded
-//    edges, gemm_bf16_tile_kernel (32 MB x 32 NB tiles) or, for a small C,
-//    gemm_bf16_kwave_kernel (16 MB x 16 NC tiles, K dealt to four waves).  A 256 x 256
+//    edges, gemm_bf16_tile_kernel (32 MB x 32 NB tiles), for a small C
+//    gemm_bf16_kwave_kernel (16 MB x 16 NC tiles, K dealt to four waves), or, for a
+//    large C of unaligned rows and a short K, gemm_bf16_kernel below.  A 256 x 256
 //    tile leaves CUs idle below 256 tiles, and unaligned rows were loaded element
 //    by element: 1000 x 3000 x 4096 159 -> 36 us, 1001 x 3001 x 4095 457 -> 71,
 //    128 x 4096 x 4096 148 -> 15, 64 x 512 x 4096 142 -> 7.4;
@@ -1133,27 +1134,39 @@ void gemm_bf16_kwave_kernel(const uint16_t* __restrict__ A, const uint16_t* __re
 constexpr size_t SMEM_BYTES = 4 * TILE_ELEMS * sizeof(uint16_t);   // 147456
 
 // The tiles that a shape can run on, and what one costs: rounds of 256 tiles, each
-// c0 + c1 us per 32 k (measured on MI355X; `odd`: K or N odd, or a pointer off a
-// 4-byte boundary).  The launcher takes the cheapest.  Large tiles move the fewest
+// c0 + c1 us per 32 k.  The launcher takes the cheapest.  Large tiles move the fewest
 // bytes per product; small ones fill the chip when C is small, and finish sooner
 // when K is short.
-enum TileKind { TILE_EDGE, TILE_GRID, TILE_WAVE };
+//  * `odd`: K or N odd, or A or B off a 4-byte boundary; TILE_REG (gemm_bf16_kernel): no
+//    16-byte rows, element-wise loads;
+//  * `narrow`: more per tile where rows of C don't start on the boundary of a
+//    lane's store (16 bytes in TILE_EDGE, 8 in TILE_GRID), so that each lane stores
+//    scattered elements.  With many tiles that bounds a short K: 8192 x 8191 x 9 170 us on
+//    128 x 128 tiles, 82 on TILE_REG, whose lanes store 32 neighbours; 8192 x 8190 x 8 119
+//    on TILE_EDGE, 84 on 64 x 64 tiles (which store whole dwords), 82 on TILE_REG;
+//    7104 x 1466 x 21 34 and 24.
+// Fitted to the times of every tile on 489 shapes of 8 to 20000 rows and columns and K
+// of 4 to 8000: the choice takes 1.02 times the best tile's time in the mean and at most
+// 1.05 times gemm_bf16_kernel's (without `narrow` and TILE_REG 1.09 and 2.1).
+enum TileKind { TILE_EDGE, TILE_GRID, TILE_WAVE, TILE_REG };
 struct TileChoice {
     TileKind kind;
     uint16_t mb, nb;              // template arguments
     uint16_t tm, tn;              // rows and columns per tile
     float c0, c1, odd_c0, odd_c1; // odd_c1 = 0: not for odd shapes
+    float narrow;
 };
 constexpr TileChoice k_tiles[] = {
-    {TILE_EDGE, 0, 0, 256, 256, 5.0f, 0.62f, 0, 0},   // K a multiple of 8
-    {TILE_GRID, 8, 4, 256, 128, 3.0f, 0.50f, 0, 0},
-    {TILE_GRID, 4, 4, 128, 128, 4.0f, 0.265f, 6.0f, 0.53f},
-    {TILE_GRID, 4, 3, 128, 96, 4.0f, 0.25f, 6.0f, 0.52f},
-    {TILE_WAVE, 4, 8, 64, 128, 2.6f, 0.155f, 4.0f, 0.33f},
-    {TILE_WAVE, 4, 4, 64, 64, 1.3f, 0.115f, 3.0f, 0.25f},
-    {TILE_WAVE, 2, 4, 32, 64, 1.2f, 0.09f, 2.0f, 0.16f},
-    {TILE_WAVE, 1, 4, 16, 64, 1.2f, 0.085f, 2.0f, 0.14f},
-    {TILE_WAVE, 1, 2, 16, 32, 0.8f, 0.055f, 1.5f, 0.12f},
+    {TILE_EDGE, 0, 0, 256, 256, 6.6f, 0.58f, 0, 0, 18.0f},   // K a multiple of 8
+    {TILE_GRID, 8, 4, 256, 128, 2.8f, 0.50f, 0, 0, 10.4f},
+    {TILE_GRID, 4, 4, 128, 128, 3.9f, 0.265f, 4.7f, 0.53f, 4.8f},
+    {TILE_GRID, 4, 3, 128, 96, 4.4f, 0.25f, 3.9f, 0.59f, 2.8f},
+    {TILE_WAVE, 4, 8, 64, 128, 3.8f, 0.155f, 4.5f, 0.37f, 0},
+    {TILE_WAVE, 4, 4, 64, 64, 1.27f, 0.125f, 2.5f, 0.245f, 0},
+    {TILE_WAVE, 2, 4, 32, 64, 1.28f, 0.10f, 2.3f, 0.165f, 0},
+    {TILE_WAVE, 1, 4, 16, 64, 0.96f, 0.088f, 2.0f, 0.165f, 0},
+    {TILE_WAVE, 1, 2, 16, 32, 1.0f, 0.055f, 1.3f, 0.12f, 0},
+    {TILE_REG, 0, 0, 256, 256, 15.7f, 1.26f, 14.6f, 3.16f, 0},
 };
 
 template <int MB, int NB, int KG, int R, bool ODD>
@@ -1189,31 +1202,34 @@ int launch_wave_tile(const uint16_t* a, const uint16_t* b, uint16_t* c, uint32_t
     return MB_OK;
 }
 
-// The cheapest tile, or nullptr: none can be launched.
-const TileChoice* choose_tile(uint32_t m, uint32_t n, uint32_t k, bool odd) {
+// The cheapest tile; `aligned`: 16-byte rows of A and B, c: where C lies.
+const TileChoice& choose_tile(uint32_t m, uint32_t n, uint32_t k, bool odd, bool aligned, uintptr_t c) {
     const TileChoice* best = nullptr;
     float least = 0.f;
     for (const TileChoice& t : k_tiles) {
-        if (odd ? t.odd_c1 == 0.f : t.kind == TILE_EDGE && k % 8) continue;
+        const bool slow = t.kind == TILE_REG ? !aligned : odd;
+        if (slow ? t.odd_c1 == 0.f : t.kind == TILE_EDGE && k % 8) continue;
         const uint64_t tiles = (uint64_t)cdiv(m, t.tm) * cdiv(n, t.tn);
-        if (tiles >= 1u << 23) continue;   // 2^32 threads or more (512 to a tile) cannot be launched
+        if (tiles >= 1u << 23) continue;   // 2^32 threads or more (512 to a tile; none of TILE_REG) cannot be launched
+        const bool narrow = t.kind == TILE_EDGE ? (n & 7) || (c & 15) : (n & 3) || (c & 7);
         const float cost = (float)((tiles + 255) / 256) *
-                           (odd ? t.odd_c0 + t.odd_c1 * cdiv(k, 32) : t.c0 + t.c1 * cdiv(k, 32));
+                           ((slow ? t.odd_c0 + t.odd_c1 * cdiv(k, 32) : t.c0 + t.c1 * cdiv(k, 32)) +
+                            (narrow ? t.narrow : 0.f));
         if (!best || cost < least) { best = &t; least = cost; }
     }
-    return best;
+    return *best;
 }
 
-int launch_tiles(const TileChoice* best, const uint16_t* a, const uint16_t* b, uint16_t* c, uint32_t m,
-                 uint32_t n, uint32_t k, bool odd, hipStream_t s) {
-    if (best->kind == TILE_EDGE) {
+int launch_tile(const TileChoice& t, const uint16_t* a, const uint16_t* b, uint16_t* c, uint32_t m,
+                uint32_t n, uint32_t k, bool odd, hipStream_t s) {
+    if (t.kind == TILE_EDGE) {
         const uint32_t tm = cdiv(m, BM), tn = cdiv(n, BN);
         hipLaunchKernelGGL(gemm_bf16_full_kernel<true>, dim3(tm * tn), dim3(256), 0, s, a, b, c, m, n, k,
                            tm, tn);
         MB_LAUNCH_CHECK("matmul_bf16");
         return MB_OK;
     }
-    switch (100 * best->kind + 10 * best->mb + best->nb) {
+    switch (100 * t.kind + 10 * t.mb + t.nb) {
         case 100 * TILE_GRID + 84: return launch_grid_tile<8, 4, 1, 3, false>(a, b, c, m, n, k, s);
         case 100 * TILE_GRID + 44: return odd ? launch_grid_tile<4, 4, 2, 4, true>(a, b, c, m, n, k, s)
                                               : launch_grid_tile<4, 4, 2, 4, false>(a, b, c, m, n, k, s);
@@ -1258,7 +1274,8 @@ int launch_gemm_bf16(const uint16_t* a, const uint16_t* b, uint16_t* c, uint32_t
     }
     if (tiles) {
         const bool odd = ((k | n) & 1) || ((((uintptr_t)a) | ((uintptr_t)b)) & 3);
-        if (const TileChoice* t = choose_tile(m, n, k, odd)) return launch_tiles(t, a, b, c, m, n, k, odd, s);
+        const TileChoice& t = choose_tile(m, n, k, odd, aligned, (uintptr_t)c);
+        if (t.kind != TILE_REG) return launch_tile(t, a, b, c, m, n, k, odd, s);
     }
     static bool attr_set[3] = {false, false, false};
     auto go = [&](auto kernel, int mode) -> int {

@@ -84,33 +84,42 @@ def run_bound(metal_function: str, inputs, outputs, scalars, dtype="f32"):
 # boundary.  One past or one short of a tile in M and N, and K of a single short stage,
 # a few stages with a remainder, and many.
 BF16_TILE_SHAPES = [
-    ((1537, 4610, 8), ("EDGE", 0, 0), ("GRID", 4, 4)),
-    ((1537, 4610, 392), ("EDGE", 0, 0), ("GRID", 4, 4)),
-    ((513, 3586, 2), ("GRID", 8, 4), ("GRID", 4, 3)),
-    ((769, 4610, 290), ("GRID", 8, 4), ("WAVE", 4, 8)),
-    ((513, 4990, 130), ("GRID", 4, 4), ("GRID", 4, 4)),
-    ((513, 4990, 290), ("GRID", 4, 4), ("GRID", 4, 4)),
-    ((513, 4990, 514), ("GRID", 4, 4), ("GRID", 4, 4)),
-    ((513, 4990, 1), None, ("GRID", 4, 4)),
-    ((513, 4990, 289), None, ("GRID", 4, 4)),
-    ((385, 4702, 130), ("GRID", 4, 3), ("GRID", 4, 3)),
-    ((385, 4702, 514), ("GRID", 4, 3), ("GRID", 4, 3)),
-    ((385, 4702, 1), None, ("GRID", 4, 3)),
-    ((385, 4701, 513), None, ("GRID", 4, 3)),
-    ((2367, 386, 2), ("WAVE", 4, 8), ("WAVE", 4, 8)),
+    ((4353, 3326, 136), ("EDGE", 0, 0), ("REG", 0, 0)),
+    ((2817, 4354, 296), ("EDGE", 0, 0), ("REG", 0, 0)),
+    ((513, 3588, 2), ("GRID", 8, 4), ("GRID", 4, 3)),
+    ((769, 4612, 130), ("GRID", 8, 4), ("WAVE", 4, 8)),
+    ((769, 4612, 290), ("GRID", 8, 4), ("WAVE", 4, 8)),
+    ((385, 4732, 130), ("GRID", 4, 4), ("GRID", 4, 3)),
+    ((385, 4732, 290), ("GRID", 4, 4), ("GRID", 4, 3)),
+    ((385, 4732, 514), ("GRID", 4, 4), ("GRID", 4, 4)),
+    ((513, 4988, 1), None, ("GRID", 4, 4)),
+    ((513, 4988, 289), None, ("GRID", 4, 4)),
+    ((385, 4732, 513), None, ("GRID", 4, 4)),
+    ((1407, 2206, 290), ("GRID", 4, 3), ("GRID", 4, 3)),
+    ((1407, 2206, 514), ("GRID", 4, 3), ("GRID", 4, 3)),
+    ((257, 3268, 1), None, ("GRID", 4, 3)),
+    ((2305, 772, 129), None, ("GRID", 4, 3)),
+    ((385, 4703, 513), None, ("GRID", 4, 3)),
+    ((257, 3586, 450), ("WAVE", 4, 8), ("WAVE", 4, 8)),
     ((193, 4098, 1026), ("WAVE", 4, 8), ("WAVE", 2, 4)),
-    ((2367, 385, 1), None, ("WAVE", 4, 8)),
-    ((2367, 385, 1025), None, ("WAVE", 4, 8)),
-    ((2049, 194, 2), ("WAVE", 4, 4), ("WAVE", 4, 4)),
-    ((2049, 194, 1026), ("WAVE", 4, 4), ("WAVE", 4, 4)),
-    ((2049, 193, 1025), None, ("WAVE", 4, 4)),
-    ((1025, 194, 2), ("WAVE", 2, 4), ("WAVE", 2, 4)),
-    ((1025, 194, 1026), ("WAVE", 2, 4), ("WAVE", 2, 4)),
-    ((1025, 193, 1025), None, ("WAVE", 2, 4)),
-    ((17, 4098, 2), ("WAVE", 1, 4), ("WAVE", 1, 4)),
-    ((17, 4098, 1026), ("WAVE", 1, 4), ("WAVE", 1, 4)),
-    ((17, 4097, 1025), None, ("WAVE", 1, 4)),
-    ((1, 2, 2), ("WAVE", 1, 2), ("WAVE", 1, 2)),
+    ((193, 4097, 1), None, ("WAVE", 4, 8)),
+    ((257, 3585, 513), None, ("WAVE", 4, 8)),
+    ((257, 3585, 1025), None, ("WAVE", 4, 8)),
+    ((129, 3266, 2), ("WAVE", 4, 4), ("WAVE", 4, 4)),
+    ((1663, 258, 290), ("WAVE", 4, 4), ("WAVE", 4, 4)),
+    ((1663, 258, 1026), ("WAVE", 4, 4), ("WAVE", 4, 4)),
+    ((1663, 257, 1025), None, ("WAVE", 4, 4)),
+    ((831, 258, 2), ("WAVE", 2, 4), ("WAVE", 2, 4)),
+    ((831, 258, 1026), ("WAVE", 2, 4), ("WAVE", 2, 4)),
+    ((831, 257, 1025), None, ("WAVE", 2, 4)),
+    ((1, 2, 2), ("WAVE", 1, 4), ("WAVE", 1, 2)),
+    ((33, 2748, 290), ("WAVE", 1, 4), ("WAVE", 1, 4)),
+    ((33, 2748, 1026), ("WAVE", 1, 4), ("WAVE", 1, 4)),
+    ((33, 2748, 1025), None, ("WAVE", 1, 4)),
+    ((1, 2, 130), ("WAVE", 1, 2), ("WAVE", 1, 2)),
     ((33, 66, 1026), ("WAVE", 1, 2), ("WAVE", 1, 2)),
+    ((1, 1, 1), None, ("WAVE", 1, 2)),
     ((33, 65, 1025), None, ("WAVE", 1, 2)),
+    ((2817, 4354, 2), ("REG", 0, 0), ("REG", 0, 0)),
+    ((1793, 3329, 1), None, ("REG", 0, 0)),
 ]

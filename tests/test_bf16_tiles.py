@@ -21,15 +21,18 @@ def _table():
 
 
 def _choose(m, n, k, odd):
+    """The tile for A and B on (odd: off) and C on a 16-byte boundary."""
     best = None
-    for kind, mb, nb, tm, tn, c0, c1, odd_c0, odd_c1 in _table():
-        if odd_c1 == 0 if odd else kind == "EDGE" and k % 8:
+    for kind, mb, nb, tm, tn, c0, c1, odd_c0, odd_c1, narrow in _table():
+        slow = odd or k % 8 or n % 8 if kind == "REG" else odd
+        if odd_c1 == 0 if slow else kind == "EDGE" and k % 8:
             continue
         tiles = -(-m // tm) * -(-n // tn)
         if tiles >= 1 << 23:
             continue
-        base, step = (odd_c0, odd_c1) if odd else (c0, c1)
-        cost = np.float32((tiles + 255) // 256) * (base + step * np.float32(-(-k // 32)))
+        base, step = (odd_c0, odd_c1) if slow else (c0, c1)
+        more = narrow if n % (8 if kind == "EDGE" else 4) else np.float32(0)
+        cost = np.float32((tiles + 255) // 256) * (base + step * np.float32(-(-k // 32)) + more)
         if best is None or cost < best[0]:
             best = (cost, (kind, mb, nb))
     return best[1]
@@ -45,6 +48,6 @@ def test_shapes_take_the_tiles_they_are_listed_for():
 
 def test_every_tile_is_listed():
     table = _table()
-    assert len(table) >= 9
+    assert len(table) >= 10
     assert {e for _, e, _ in BF16_TILE_SHAPES if e} == {r[:3] for r in table}
     assert {o for _, _, o in BF16_TILE_SHAPES} == {r[:3] for r in table if r[8] != 0}

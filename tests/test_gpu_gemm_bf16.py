@@ -105,15 +105,13 @@ def test_kernel_attrs_report_register_split(mb):
         assert attrs["arch_vgprs"] > 0 and 1 <= attrs["waves_per_simd"] <= 8, (name, attrs)
 
 
-# Shapes away from full 256 x 256 tiles: each kind of tile, one past and one short
-# of a tile, of a 32-deep stage and of a chunk of 8, even and odd rows.
+# Shapes away from full 256 x 256 tiles: ragged and odd sizes, one past and one short
+# of a tile, of a 32-deep stage and of a chunk of 8, even and odd rows.  (Every tile by
+# itself: test_matmul_bf16_every_tile.)
 @pytest.mark.parametrize("m,n,k", [
-    (3001, 3002, 136),                              # guarded 256 x 256 tiles
-    (2815, 2900, 72), (3000, 3002, 70), (2049, 3970, 250), (1000, 3000, 98),   # 256 x 128
-    (1025, 2050, 322), (1001, 3001, 97),            # 128 x 96, even and odd rows
-    (1023, 2047, 289),                              # 64 x 128, odd rows
-    (513, 1026, 130), (511, 1023, 131),             # 64 x 64, 32 x 64 odd rows
-    # 16 x 32
+    (3001, 3002, 136), (2815, 2900, 72), (3000, 3002, 70), (2049, 3970, 250),
+    (1025, 2050, 322), (1000, 3000, 98), (1001, 3001, 97), (1023, 2047, 289),
+    (513, 1026, 130), (511, 1023, 131),
     (33, 66, 34), (31, 65, 33), (130, 200, 1026), (129, 199, 1025),
     (17, 34, 2), (15, 33, 1), (16, 30, 4098), (17, 31, 4097),
 ])
