@@ -42,7 +42,7 @@ constexpr int SA = BK + 4;   // As (and transposed Bs) row stride (floats)
 constexpr int SB = BN + 4;   // Bs row stride (floats)
 
 // Operands of 2 GB or more and C rows of more than 8 million columns, which 32-bit buffer
-// offsets do not reach (and K = 0): fp32 MFMA, element-wise guarded loads through 64-bit addresses.
+// offsets do not reach, a short K with few tiles, and K = 0: fp32 MFMA, element-wise guarded loads through 64-bit addresses.
 //  * BK = 64 per stage, LDS double buffered, one barrier per stage; operands
 //    are register-staged two stages ahead;
 //  * 4 waves own a 2x2 grid of 32x32 sub-tiles (v_mfma_f32_32x32x2f32);
@@ -606,8 +606,15 @@ int launch_variant(const GemmF32Args& g, uint32_t batch, hipStream_t s, bool f32
     // of the waves without a unit, are faster here too: 2048 x 2048 x 16 10.8 us against
     // 17.1 for register-staged fp32 MFMA tiles, x 64 12.8 and 16.9, 4096 x 4096 x 32 35.4
     // and 56.6, 100 x 60000 x 64 20.8 and 28.7.
+    // But at most one tile per CU and K in one or two of the 16-deep units (or, up to 64
+    // tiles, in four, one 64-deep stage) are left to the element-wise kernel below, where
+    // nothing is split and one exchange of partial tiles is shorter: 1 x 1 x 1 3.7 us, 4.1
+    // split; 1000 x 1000 x 8 4.8 and 5.2; 500 x 1000 x 31 4.85 and 4.92 (x 47 5.4 and 5.1);
+    // 1 x 4000 x 63 4.5 and 4.7 (x 65 5.6 and 5.1).
+    const uint64_t all = nblocks * batch;
+    const bool tiny = (g.k <= 32 && all <= 256) || (g.k <= (uint32_t)BK && all <= 64);
     const uint64_t c_bytes = (uint64_t)std::min(g.m, 64u) * std::max(g.ldc, g.ldr) * 4;
-    if (g.k > 0 && (uint64_t)g.m * g.lda * 4 < 0x80000000ull && b_rows * g.ldb * 4 < 0x80000000ull &&
+    if (g.k > 0 && !tiny && (uint64_t)g.m * g.lda * 4 < 0x80000000ull && b_rows * g.ldb * 4 < 0x80000000ull &&
         c_bytes < 0x80000000ull) {
         GemmF32Args q = g;
         q.tiles_n = cdiv(g.n, EPI == EPI_SWIGLU ? 32 : 64);

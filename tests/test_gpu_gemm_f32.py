@@ -102,6 +102,26 @@ def test_matmul_f32_split_edges(mb, dev, m, n, k, shift):
     assert np.all(c[:shift] == 7.0) and np.all(c[shift + m * n:] == 7.0)
 
 
+# K up to 32 with at most 256 tiles, and up to 64 with 64, run element-wise on fp32
+# MFMA, other short K on the split kernel: both sides of these lines, one past and one
+# short of a unit
+@pytest.mark.parametrize("m,n,k", [(1027, 1025, 1), (1090, 1030, 7), (1100, 1030, 15), (1026, 1100, 33),
+                                   (1024, 1023, 32), (1024, 1023, 33), (513, 511, 64), (511, 513, 63),
+                                   (509, 511, 65), (16321, 2, 18), (2, 16399, 31), (1, 1, 1)])
+def test_matmul_f32_short_k(mb, dev, m, n, k):
+    """Every product is added with a rounding of at most 2^-24 of a partial sum (on the
+    split kernel less often, see above), and no partial sum is above sum |a b|."""
+    a, b = seeded(m + k, (m, k)), seeded(n + k, (k, n))
+    buf = torch.full((m * n + 8,), 7.0, device=dev)
+    d_a, d_b = a.to(dev), b.to(dev)
+    launch("mb_launch_matmul_f32", ptr(d_a), ptr(d_b), ptr(buf), m, n, k, None)
+    c = buf.cpu().numpy()
+    A, B = a.numpy().astype(np.float64), b.numpy().astype(np.float64)
+    bound = max(2.0 ** -22, k * 2.0 ** -24) * (np.abs(A) @ np.abs(B))
+    assert np.all(np.abs(c[:m * n].reshape(m, n) - A @ B) <= bound)
+    assert np.all(c[m * n:] == 7.0)
+
+
 @pytest.mark.parametrize("m,n,k", [(70, 67, 129), (128, 192, 640)])
 def test_matmul_f32_values_the_split_cannot_hold(mb, dev, m, n, k):
     """Infinities, NaN, values that round to a bf16 infinity, and rows or columns
@@ -147,20 +167,21 @@ def test_matmul_f32_operand_past_2gb(mb, dev):
 # term of the split has to survive, whatever stands beside it.
 @pytest.mark.parametrize("e", [-100, -110, -115, -120, -126, -130, -140, -149])
 def test_matmul_f32_small_elements_keep_their_bits(mb, dev, e):
-    """A = [1, v], B = [0; w]: the product v w alone, v from 2^e on and w = 2^100 (or the
+    """A = [1, 0 .., v], B = [0; ..; w]: the product v w alone, v from 2^e on and w = 2^100 (or the
     other way round).  Both are powers of two or 24-bit numbers, so fp32 products would
     be exact up to one rounding; a subnormal v has the bits fp32 holds."""
     v = np.float32(1.37 * 2.0 ** e)
-    for n in (1, 2, 65):
-        a = torch.tensor([[1.0, float(v)]])
-        b = torch.zeros((2, n))
-        b[1] = 2.0 ** 100
+    for n, k in ((1, 2), (65, 2), (1, 66), (2, 67), (65, 68)):   # (K = 2: fp32 MFMA)
+        a = torch.zeros((1, k))
+        a[0, 0], a[0, k - 1] = 1.0, float(v)
+        b = torch.zeros((k, n))
+        b[k - 1] = 2.0 ** 100
         want = float(v) * 2.0 ** 100
         for x, y in ((a, b), (b.T.contiguous(), a.T.contiguous())):
             d_x, d_y = x.to(dev), y.to(dev)
             m, nn = x.shape[0], y.shape[1]
             d_c = torch.zeros((m, nn), device=dev)
-            launch("mb_launch_matmul_f32", ptr(d_x), ptr(d_y), ptr(d_c), m, nn, 2, None)
+            launch("mb_launch_matmul_f32", ptr(d_x), ptr(d_y), ptr(d_c), m, nn, k, None)
             got = d_c.cpu().numpy().astype(np.float64)
             assert np.all(np.abs(got - want) <= 2.0 ** -23 * want), (n, got.ravel()[0] / want - 1)
 
