@@ -1,4 +1,5 @@
-// conv2d as an implicit GEMM on fp32 MFMA: NHWC input, OHWI weight, NHWC output.
+// conv2d as an implicit GEMM on MFMA (fp32 as bf16 terms, or fp32): NHWC input, OHWI
+// weight, NHWC output.
 //
 // Spec: reference mlx/kernels/common/conv2d.py:11-12 (mx.conv2d: cross-
 // correlation, dilation 1, groups 1), registry mlx/kernels/common/registry.py:
@@ -19,7 +20,7 @@
 //    the tap is uniform per stage and each A row is one contiguous 128-byte NHWC
 //    channel run, fetched by DMA straight into LDS or zero-filled at the image
 //    border.  Tiles are 32 pixels x 64 channels (details at the kernel);
-//  * operands past 2 GB, and K <= 32 with few tiles (conv2d_f32_kernel): 64 x 64 tiles with 8 waves, both
+//  * operands past 2 GB, and most K <= 32 with C % 32 != 0 (conv2d_f32_kernel): 64 x 64 tiles with 8 waves, both
 //    operands gathered element-wise through 64-bit addresses, staged two stages
 //    ahead in registers and stored K-contiguous in LDS (row stride 36 floats: 16
 //    lanes reading 16 consecutive rows with ds_read_b128 cover all 64 banks once),
@@ -562,10 +563,14 @@ int launch_conv2d(const float* x, const float* w, float* y, uint32_t n, uint32_t
     //    over 15x30x65x64 10.1 us, split 13.1; 28x28x64 3x3 7.5 and 10.2);
     //  * split tiles, one workgroup per CU 4.5 + 0.17 u, two 8 + 0.31 u: all else
     //    (8x30x30x128 -> 96 3x3 17.5 us, fp32 MFMA 22.1; 8x64x64x64 -> 128 34.9 and 40.8);
-    //  * element-wise fp32 MFMA: K in one 32-deep stage and at most one tile per CU, where
-    //    the split kernel's waves have a unit or none each (2x40x40x3 -> 64 3x3 4.7 us on
-    //    5.4, 21x5x71x16 -> 32 1x1 4.7 on 4.9; 24x90x90x16 -> 64 1x1 26.3 on 16.2).
-    const bool tiny = !fast && sh.k <= (uint32_t)BK && nblocks <= 256;
+    //  * element-wise fp32 MFMA: K in one 32-deep stage, where the split kernel's waves
+    //    have a unit or none each, with at most one tile per CU (2x40x40x3 -> 64 3x3 4.7 us on
+    //    5.4, 21x5x71x16 -> 32 1x1 4.7 on 4.9), with a DMA per element (C no multiple of 4:
+    //    24x90x90x3 -> 64 3x3 26.4 on 34.5, 24x90x90x1 -> 64 1x1 20.3 on 29.1) or with two
+    //    units (24x90x90x20 -> 64 1x1 26.1 on 28.3).  One unit of 16-byte chunks and many
+    //    tiles: 8x90x90x8 -> 64 1x1 11.6 on 10.8, 24 images 26.3 on 26.2.  From K = 36 on
+    //    the split: 24x90x90x4 -> 64 3x3 40.1 on 29.7.
+    const bool tiny = !fast && sh.k <= (uint32_t)BK && (nblocks <= 256 || c % 4 || sh.k > 16);
     if (near && !tiny) {
         const float u = (float)cdiv(sh.k, 16);
         const float by_split = nblocks <= 256 ? 4.5f + 0.17f * u

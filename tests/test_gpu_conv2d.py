@@ -80,6 +80,9 @@ def test_conv2d_registry_config(mb, name):
     (24, 60, 61, 4, 8, 1, 1, 1, 0), (24, 60, 61, 3, 65, 3, 3, 1, 1), (23, 60, 60, 20, 66, 2, 3, 1, 1),
     (3, 301, 303, 3, 40, 7, 7, 1, 3), (24, 60, 60, 36, 32, 1, 1, 1, 0), (7, 230, 119, 12, 30, 3, 3, 2, 1),
     (2, 17, 19, 36, 130, 3, 3, 1, 1), (3, 9, 9, 7, 64, 1, 1, 1, 0), (1, 40, 30, 6, 20, 5, 3, 2, 2),
+    # K <= 32 (element-wise unless one unit of whole chunks) and just past it
+    (24, 60, 61, 5, 65, 3, 3, 1, 1), (24, 50, 50, 11, 64, 1, 3, 1, 0), (24, 50, 51, 20, 40, 1, 1, 1, 0),
+    (24, 50, 51, 16, 40, 1, 1, 1, 0), (24, 50, 51, 2, 40, 3, 5, 1, 1),
 ])
 def test_conv2d_split_shapes(mb, dev, n, h, w, c, o, r, s, st, pad):
     """A sum is added up in 6 steps per 16 k (and 3 for the waves' parts), each rounding
@@ -99,7 +102,7 @@ def test_conv2d_split_shapes(mb, dev, n, h, w, c, o, r, s, st, pad):
     assert torch.all(d_y[n * p * q * o:] == 7.0)
 
 
-@pytest.mark.parametrize("n,c", [(24, 4), (24, 3), (1, 4), (1, 3)])
+@pytest.mark.parametrize("n,c", [(24, 4), (24, 3), (24, 5), (1, 4), (1, 3)])
 def test_conv2d_values_the_split_cannot_hold(mb, dev, n, c):
     """Infinities, NaN and channels near the smallest normal number."""
     h = w = 60
@@ -122,7 +125,7 @@ def test_conv2d_values_the_split_cannot_hold(mb, dev, n, c):
     assert np.all(np.abs(got[fin] - want[fin]) <= (2.0 ** -20 * size)[fin])
 
 
-@pytest.mark.parametrize("c", [4, 3, 64])
+@pytest.mark.parametrize("c", [4, 3, 5, 64])
 def test_conv2d_small_weights_keep_their_bits(mb, dev, c):
     """A patch that a ReLU left at zero except under one tiny weight: the outputs are
     that product alone, exact up to one rounding (the bound leaves room for one more)."""
