@@ -227,6 +227,47 @@ def test_attention_tile_edges(mb, s, d, h, hkv):
     assert (np.abs(f64(y) - (f64(x) + attn)) <= 2.0 ** -22 * (np.abs(f64(x)) + np.abs(attn))).all()
 
 
+@pytest.mark.parametrize("dh", [32, 64, 128])
+def test_attention_scores_are_summed_in_short_chains(mb, dh):
+    """No further from 64 bits than q.k in four interleaved fp32 chains and p.v in one, in
+    the mean over ten inputs.  q, k and v are columns of x (projections of ones and zeros,
+    so exact); the tenth allowed above is for the spread of a mean over ten."""
+    s, got_sq, chains_sq = 62, 0.0, 0.0
+    eye = np.eye(dh, dtype=np.float32)
+    w = torch.from_numpy(np.concatenate([eye, eye[:, ::-1], eye], 1).copy())
+    ang = np.arange(s)[:, None] * 10000.0 ** (-np.arange(0, dh, 2) / dh)
+    cos, sin = np.cos(ang).astype(np.float32), np.sin(ang).astype(np.float32)
+
+    def fma(a, b, c):
+        return (a.astype(np.float64) * b + c).astype(np.float32)
+
+    def rope(t):
+        a, b = t[:, 0::2], t[:, 1::2]
+        return np.stack((fma(a, cos, -(b * sin)), fma(a, sin, b * cos)), -1).reshape(s, dh)
+
+    for seed in range(10):
+        x = seeded(80 + seed, (s, dh))
+        (y,) = run_bound("llama_attention_f32", [(0, x), (1, w), (2, torch.from_numpy(eye))], [(3, (s, dh))],
+                         [(4, "u32", s), (5, "u32", dh), (6, "u32", 1), (7, "u32", 1), (8, "f32", 10000.0)])
+        want = oracle.llama_attention(f64(x), f64(w), eye.astype(np.float64), n_heads=1, n_kv_heads=1)
+        v = x.numpy()
+        q, k = rope(v), rope(v[:, ::-1])
+        part = [np.zeros((s, s), np.float32) for _ in range(4)]
+        for d in range(dh):
+            part[d % 4] = fma(q[:, d, None], k[None, :, d], part[d % 4])
+        sc = ((part[0] + part[1]) + (part[2] + part[3])) * np.float32(dh ** -0.5)
+        p = np.exp(sc - sc.max(1, keepdims=True))
+        out = np.zeros((s, dh), np.float32)
+        for j in range(s):
+            out = fma(p[:, j, None], v[None, j], out)
+        out /= p.sum(1, keepdims=True, dtype=np.float32)
+        got_sq += ((f64(y) - want) ** 2).sum()
+        chains_sq += ((out - want) ** 2).sum()
+    ratio = (got_sq / chains_sq) ** 0.5
+    print("error over that of the chains: %.3f" % ratio, flush=True)
+    assert ratio <= 1.1
+
+
 def test_rejects_bad_shapes(mb):
     import ctypes  # noqa: F401
     from metalbench_amd import native
