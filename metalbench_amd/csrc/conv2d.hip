@@ -482,8 +482,8 @@ struct ImageLoad {
     }
 };
 
-// 64 pixels x 64 channels, the waves dividing K.  32x56x56x64 -> 64 3x3: 55-56 us (fp32 MFMA
-// 61.8); 16x224x224x3 -> 64 7x7: 57 us (element-wise loads on fp32 MFMA 83.8).  What a
+// 64 pixels x 64 channels, the waves dividing K.  32x56x56x64 -> 64 3x3: 56-58 us by card
+// (fp32 MFMA 62-63); 16x224x224x3 -> 64 7x7: 57.5 us (element-wise loads on fp32 MFMA 83.9).  What a
 // tile costs beside its MFMAs is its start (first fetch, first split) and end (four
 // partial tiles through LDS), for nine units per wave here.
 // (256-pixel tiles, a wave per 64 pixels over all of K with B's terms shared, ran 50 and

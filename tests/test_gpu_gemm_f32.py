@@ -80,8 +80,9 @@ def test_matmul_registry_config(mb, name):
 
 
 # The split kernel's edges (64 x 64 tiles, 16-deep k units dealt to 4 waves, two
-# LDS slots per wave): one past and one short of a tile and of a unit, 1 to 4
-# units per wave, a wave without units.
+# LDS slots per wave): one past and one short of a tile and of a unit, 1 to 8 units per
+# wave.  (In so few tiles K up to 64 runs element-wise on fp32 MFMA: the first three;
+# waves without a unit: test_matmul_f32_short_k.)
 @pytest.mark.parametrize("m,n,k", [(65, 63, 15), (63, 65, 17), (64, 64, 48), (129, 66, 65),
                                    (66, 127, 129), (1, 2, 191), (130, 1, 257), (200, 333, 512)])
 @pytest.mark.parametrize("shift", [0, 1])
