@@ -606,13 +606,14 @@ int launch_variant(const GemmF32Args& g, uint32_t batch, hipStream_t s, bool f32
     // of the waves without a unit, are faster here too: 2048 x 2048 x 16 10.8 us against
     // 17.1 for register-staged fp32 MFMA tiles, x 64 12.8 and 16.9, 4096 x 4096 x 32 35.4
     // and 56.6, 100 x 60000 x 64 20.8 and 28.7.
-    // But at most one tile per CU and K in one or two of the 16-deep units (or, up to 64
-    // tiles, in four, one 64-deep stage) are left to the element-wise kernel below, where
+    // But at most one tile per CU and K up to 36, little more than two of the 16-deep units
+    // (or, up to 64 tiles, in four, one 64-deep stage), are left to the element-wise kernel below, where
     // nothing is split and one exchange of partial tiles is shorter: 1 x 1 x 1 3.7 us, 4.1
-    // split; 1000 x 1000 x 8 4.8 and 5.2; 500 x 1000 x 31 4.85 and 4.92 (x 47 5.4 and 5.1);
+    // split; 1000 x 1000 x 8 4.8 and 5.2; 1021 x 1021 x 33 5.25 and 5.58, x 36 5.38 and 5.56;
+    // 960 x 762 x 36 5.24 and 5.29, x 40 5.37 and 5.29, x 47 5.67 and 5.30;
     // 1 x 4000 x 63 4.5 and 4.7 (x 65 5.6 and 5.1).
     const uint64_t all = nblocks * batch;
-    const bool tiny = (g.k <= 32 && all <= 256) || (g.k <= (uint32_t)BK && all <= 64);
+    const bool tiny = (g.k <= 36 && all <= 256) || (g.k <= (uint32_t)BK && all <= 64);
     const uint64_t c_bytes = (uint64_t)std::min(g.m, 64u) * std::max(g.ldc, g.ldr) * 4;
     if (g.k > 0 && !tiny && (uint64_t)g.m * g.lda * 4 < 0x80000000ull && b_rows * g.ldb * 4 < 0x80000000ull &&
         c_bytes < 0x80000000ull) {

@@ -103,11 +103,11 @@ def test_matmul_f32_split_edges(mb, dev, m, n, k, shift):
     assert np.all(c[:shift] == 7.0) and np.all(c[shift + m * n:] == 7.0)
 
 
-# K up to 32 with at most 256 tiles, and up to 64 with 64, run element-wise on fp32
+# K up to 36 with at most 256 tiles, and up to 64 with 64, run element-wise on fp32
 # MFMA, other short K on the split kernel: both sides of these lines, one past and one
 # short of a unit
 @pytest.mark.parametrize("m,n,k", [(1027, 1025, 1), (1090, 1030, 7), (1100, 1030, 15), (1026, 1100, 33),
-                                   (1024, 1023, 32), (1024, 1023, 33), (513, 511, 64), (511, 513, 63),
+                                   (1024, 1023, 32), (1024, 1023, 33), (1021, 1021, 36), (1021, 1021, 37), (513, 511, 64), (511, 513, 63),
                                    (509, 511, 65), (16321, 2, 18), (2, 16399, 31), (1, 1, 1)])
 def test_matmul_f32_short_k(mb, dev, m, n, k):
     """Every product is added with a rounding of at most 2^-24 of a partial sum (on the
