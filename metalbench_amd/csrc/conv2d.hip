@@ -567,10 +567,14 @@ int launch_conv2d(const float* x, const float* w, float* y, uint32_t n, uint32_t
     //    have a unit or none each, with at most one tile per CU (2x40x40x3 -> 64 3x3 4.7 us on
     //    5.4, 21x5x71x16 -> 32 1x1 4.7 on 4.9), with a DMA per element (C no multiple of 4:
     //    24x90x90x3 -> 64 3x3 26.4 on 34.5, 24x90x90x1 -> 64 1x1 20.3 on 29.1) or with two
-    //    units (24x90x90x20 -> 64 1x1 26.1 on 28.3).  One unit of 16-byte chunks and many
-    //    tiles: 8x90x90x8 -> 64 1x1 11.6 on 10.8, 24 images 26.3 on 26.2.  From K = 36 on
-    //    the split: 24x90x90x4 -> 64 3x3 40.1 on 29.7.
-    const bool tiny = !fast && sh.k <= (uint32_t)BK && (nblocks <= 256 || c % 4 || sh.k > 16);
+    //    units (24x90x90x20 -> 64 1x1 26.1 on 28.3).  One unit of 16-byte chunks gains by the
+    //    split where the last of few rounds of 256 tiles is the second on its CUs, whose
+    //    workgroups hide each other's ends: 257 to 512 tiles 6.4-7.4 on 5.4-6.2, 769 to 1024
+    //    11.3 on 10.5; between and beyond it loses (513 to 768 9.1 on 9.4, 1200 12.5 on 13.0,
+    //    19840 145 on 165).  From K = 36 on the split: 24x90x90x4 -> 64 3x3 40.1 on 29.7.
+    const uint64_t rounds = (nblocks + 255) / 256;
+    const bool one_unit = c % 4 == 0 && sh.k <= 16 && (rounds == 2 || rounds == 4);
+    const bool tiny = !fast && sh.k <= (uint32_t)BK && !one_unit;
     if (near && !tiny) {
         const float u = (float)cdiv(sh.k, 16);
         const float by_split = nblocks <= 256 ? 4.5f + 0.17f * u

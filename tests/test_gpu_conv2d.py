@@ -80,7 +80,9 @@ def test_conv2d_registry_config(mb, name):
     (24, 60, 61, 4, 8, 1, 1, 1, 0), (24, 60, 61, 3, 65, 3, 3, 1, 1), (23, 60, 60, 20, 66, 2, 3, 1, 1),
     (3, 301, 303, 3, 40, 7, 7, 1, 3), (24, 60, 60, 36, 32, 1, 1, 1, 0), (7, 230, 119, 12, 30, 3, 3, 2, 1),
     (2, 17, 19, 36, 130, 3, 3, 1, 1), (3, 9, 9, 7, 64, 1, 1, 1, 0), (1, 40, 30, 6, 20, 5, 3, 2, 2),
-    # K <= 32 (element-wise unless one unit of whole chunks) and just past it
+    # K <= 32 (element-wise, unless one unit of whole chunks in the second or fourth round
+    # of 256 tiles: 458, 1024 and, further down, 957 of them) and just past it
+    (8, 60, 61, 4, 8, 1, 1, 1, 0), (16, 64, 64, 8, 64, 1, 1, 1, 0),
     (24, 60, 61, 5, 65, 3, 3, 1, 1), (24, 50, 50, 11, 64, 1, 3, 1, 0), (24, 50, 51, 20, 40, 1, 1, 1, 0),
     (24, 50, 51, 16, 40, 1, 1, 1, 0), (24, 50, 51, 2, 40, 3, 5, 1, 1),
 ])
